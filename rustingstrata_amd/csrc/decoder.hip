@@ -472,65 +472,118 @@ hipError_t launch_gemv_f32(const float* w, int rows, int cols, const float* x, u
 
 // ---- f32-weight GEMM (gemm_dense of a float matrix): each output's dot runs over k in index order with a multiply
 // then an add, as Tensor::matvec's f32 iterator sum (src/weights.rs:29-37): the CPU's bits. That makes every output
-// one dependent chain of 2 cols instructions, so the kernel is built for VALU throughput with two waves a SIMD: a
-// block of 4 waves takes 64 positions (a lane each) x 8 weight rows (2 a wave, 2 chains a lane); per step of 64 k the
-// block stages x transposed ([k][position]: a lane's reads hit distinct banks) and the 8 rows' weights in LDS, and a
-// lane reads its x value once per k and the weights as wave-wide broadcasts (one 16-byte read for 4 k of a row). ----
-constexpr int GF_M = 64, GF_RW = 4, GF_R = 4 * GF_RW, GF_K = 64;  // GF_RW rows (chains) a wave (4: 102 -> 87 us at 4096 x 128 x 2048)
+// one dependent chain of 2 cols instructions (a lone wave issues one in 5-6 cycles), so few outputs are bound by the
+// chain and many by the VALU (62 us for 4096 x 128 x 2048 at two instructions a term). Three forms by the number of
+// outputs, n rows (launch_gemm_f32); router of 128 x 2048, us a call, before (one form: 4 chains a lane, x and weights
+// through one LDS buffer whose loads each step waited for) and now: 27 tokens 72 -> 18, 512 72 -> 28, 1501 72 -> 39,
+// 4096 77 -> 68. ----
+
+// A block of 4 waves takes 64 positions (a lane each) x 4 RW weight rows (RW chains a lane). x and the weight rows come
+// by direct global-to-LDS loads into a ring of GF_NB steps of 32 k (four steps in flight: one step's work is shorter
+// than a trip to memory), the registers of a group are read from it one group ahead. x sits as [position][32 k] with
+// 16-byte chunk c of position p at c ^ ((p / 2) & 7): the 16 lanes of a 16-byte read touch every bank once.
+constexpr int GF_M = 64, GF_K = 32, GF_NB = 6;  // positions a block; k of a step; steps of x in the LDS ring
+template <int RW>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ w, int rows, int cols,
                                                        const float* __restrict__ x, uint64_t x_stride, float* y,
                                                        uint64_t y_stride, int n, int act) {
-    __shared__ __align__(16) float xs[GF_K][GF_M + 1];  // (+1: the staging writes spread over banks)
-    __shared__ __align__(16) float ws[GF_R][GF_K];
-    const int m0 = blockIdx.x * GF_M, r0 = blockIdx.y * GF_R, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    // staging: x rows m0 + tid / KQ + SP i (i < NP), k k0 + 4 (tid % KQ) .. + 3; w row r0 + tid / KQ (< GF_R)
-    constexpr int KQ = GF_K / 4, SP = 256 / KQ, NP = GF_M / SP;
-    static_assert(GF_R <= SP, "one pass stages the weight rows");
-    const int sm = tid / KQ, sk = 4 * (tid % KQ);
-    float acc[GF_RW] = {};
-    float4 xv[NP], wv;
-    auto load = [&](int k0) {
+    constexpr int GK = 32 / RW, GS = GF_K / GK;  // k of a register group; groups a step
+    constexpr int NL = GF_M * GF_K * 4 / 1024 / 4;          // load instructions a wave and step
+    __shared__ __align__(16) float xs[GF_NB][GF_M * GF_K];
+    __shared__ __align__(16) float ws[GF_NB][4 * RW * GF_K];
+    const int m0 = blockIdx.x * GF_M, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r0 = blockIdx.y * 4 * RW + RW * wave;
+    const int nst = (cols + GF_K - 1) / GF_K;
+    // load instruction i of this wave: x rows 8 (NL wave + i) + lane / 8, LDS chunk lane % 8 of the row holding its
+    // chunk (lane % 8) ^ (row % 8); rows past n read the last row, columns past the end the row's last ones (unused)
+    const float* xr[NL];
+    int xc[NL];
 #pragma unroll
-        for (int i = 0; i < NP; i++) {
-            const int m = m0 + sm + SP * i;
-            xv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (m < n && k0 + sk < cols) xv[i] = *(const float4*)(x + (uint64_t)m * x_stride + k0 + sk);
-        }
-        wv = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (sm < GF_R && r0 + sm < rows && k0 + sk < cols) wv = *(const float4*)(w + (uint64_t)(r0 + sm) * cols + k0 + sk);
+    for (int i = 0; i < NL; i++) {
+        const int r = 8 * (NL * wave + i) + (lane >> 3);
+        xr[i] = x + (uint64_t)min(m0 + r, n - 1) * x_stride;
+        xc[i] = 4 * ((lane & 7) ^ ((r >> 1) & 7));
+    }
+    const float* wr = w + (uint64_t)min(r0 + (lane >> 3), rows - 1) * cols;
+    auto issue = [&](int st, int b) __attribute__((always_inline)) {
+        const int k0 = min(st, nst - 1) * GF_K;
+#pragma unroll
+        for (int i = 0; i < NL; i++) load_lds16((uint64_t)(xr[i] + min(k0 + xc[i], cols - 4)), &xs[b][256 * (NL * wave + i)]);
+        if (lane < 8 * RW) load_lds16((uint64_t)(wr + min(k0 + 4 * (lane & 7), cols - 4)), &ws[b][RW * GF_K * wave]);
     };
-    load(0);
-    for (int k0 = 0; k0 < cols; k0 += GF_K) {
-        __syncthreads();
+    float acc[RW] = {};
+    float4 xa[2][GK / 4];
+    float4 wa[2][RW][GK / 4];
+    // the registers of group gi (k = GK gi ..): x from the step's buffer, the weights through the scalar cache
+    auto fetch = [&](int gi, int b, float4 (&xg)[GK / 4], float4 (&ww)[RW][GK / 4]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NP; i++) {
-            const int m = sm + SP * i;
-            xs[sk][m] = xv[i].x; xs[sk + 1][m] = xv[i].y; xs[sk + 2][m] = xv[i].z; xs[sk + 3][m] = xv[i].w;
-        }
-        if (sm < GF_R) *(float4*)&ws[sm][sk] = wv;
-        __syncthreads();
-        if (k0 + GF_K < cols) load(k0 + GF_K);
-        const int kn = min(GF_K, cols - k0);
-        const float* wr = &ws[GF_RW * wave][0];
-        // the whole step unrolled (cols % 4 == 0; a shorter last step ends early), so its LDS reads run ahead
+        for (int q = 0; q < GK / 4; q++) xg[q] = *(const float4*)&xs[b][lane * GF_K + 4 * (((gi % GS) * (GK / 4) + q) ^ ((lane >> 1) & 7))];
 #pragma unroll
-        for (int k = 0; k < GF_K; k += 4) {
-            if (k >= kn) break;
-            const float a[4] = {xs[k][lane], xs[k + 1][lane], xs[k + 2][lane], xs[k + 3][lane]};
-            float4 wj[GF_RW];
+        for (int j = 0; j < RW; j++)
 #pragma unroll
-            for (int j = 0; j < GF_RW; j++) wj[j] = *(const float4*)(wr + j * GF_K + k);
+            for (int q = 0; q < GK / 4; q++) ww[j][q] = *(const float4*)&ws[b][(RW * wave + j) * GF_K + (gi % GS) * GK + 4 * q];
+    };
+    auto run = [&](const float4 (&xg)[GK / 4], const float4 (&ww)[RW][GK / 4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < GK / 4; q++) {
+            const float a[4] = {xg[q].x, xg[q].y, xg[q].z, xg[q].w};
+            float p[4][RW];
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
-                for (int j = 0; j < GF_RW; j++) acc[j] += a[e] * (e == 0 ? wj[j].x : e == 1 ? wj[j].y : e == 2 ? wj[j].z : wj[j].w);
+                for (int j = 0; j < RW; j++) {
+                    const float4 wq = ww[j][q];
+                    p[e][j] = a[e] * (e == 0 ? wq.x : e == 1 ? wq.y : e == 2 ? wq.z : wq.w);
+                    if constexpr (RW == 1) asm volatile("" : "+v"(p[e][j]));
+                }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int j = 0; j < RW; j++) acc[j] += p[e][j];
         }
+    };
+    const int ng = cols / GK;
+#pragma unroll
+    for (int b = 0; b < GF_NB - 1; b++) issue(b, b);
+    wait_vm<(NL + 1) * (GF_NB - 2)>();
+    lds_barrier();
+    if (ng > 0) fetch(0, 0, xa[0], wa[0]);
+    int b = 0;
+    // one step; PAR: its first group's register set
+    auto step = [&](int st, auto PAR) __attribute__((always_inline)) {
+        constexpr int par = decltype(PAR)::value;
+        const int b1 = b + 1 == GF_NB ? 0 : b + 1, bp = b == 0 ? GF_NB - 1 : b - 1;
+        wait_vm<(NL + 1) * (GF_NB - 3)>();  // this wave's loads of step st + 1
+        lds_barrier();                // everybody's; and buffer bp (step st - 1) has been read
+        issue(st + GF_NB - 1, bp);
+#pragma unroll
+        for (int u = 0; u < GS; u++) {
+            const int gi = st * GS + u;
+            if (gi >= ng) break;
+            wait_lds();  // this group's registers (before the next group's loads: scalar loads complete out of order)
+            // (past the last group: the last one again, so that the weights stay in scalar registers)
+            fetch(gi + 1 < ng ? gi + 1 : gi, u + 1 < GS || gi + 1 >= ng ? b : b1, xa[(par + u + 1) & 1], wa[(par + u + 1) & 1]);
+            run(xa[(par + u) & 1], wa[(par + u) & 1]);
+#pragma unroll
+            for (int j = 0; j < RW; j++) asm volatile("" : "+v"(acc[j]));  // (keeps this group's work ahead of the next wait)
+        }
+        if (st + 1 == nst)  // the last columns, less than a group
+            for (int k = ng * GK; k < cols; k++)
+#pragma unroll
+                for (int j = 0; j < RW; j++)
+                    acc[j] += xs[b][lane * GF_K + 4 * (((k - st * GF_K) >> 2) ^ ((lane >> 1) & 7)) + (k & 3)] * ws[b][(RW * wave + j) * GF_K + k - st * GF_K];
+        b = b1;
+    };
+    for (int st = 0; st < nst; st += 2) {
+        step(st, std::integral_constant<int, 0>{});
+        if (st + 1 < nst) step(st + 1, std::integral_constant<int, GS & 1>{});
     }
+    wait_loads();  // (the ring's loads past the last step)
     const int m = m0 + lane;
     if (m < n) {
 #pragma unroll
-        for (int j = 0; j < GF_RW; j++) {
-            const int r = r0 + GF_RW * wave + j;
+        for (int j = 0; j < RW; j++) {
+            const int r = r0 + j;
             if (r >= rows) continue;
             float* yo = y + (uint64_t)m * y_stride + r;
             const float v = acc[j];
@@ -539,11 +592,97 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
     }
 }
 
+// Few outputs: four lanes share an output's products (lane e of a quad holds terms 4 e .. 4 e + 3 of each 16, one
+// multiply for four terms) and each of them runs the whole chain, taking the products by quad permutes that fold into
+// the adds; a wave takes 16 rows x P positions, whose chains interleave (an add may not follow its predecessor within
+// two issues), U groups of 16 terms loaded ahead.
+template <int P, int U>
+__global__ __launch_bounds__(256) void gemm_f32_quad_kernel(const float* __restrict__ w, int rows, int cols,
+                                                            const float* __restrict__ x, uint64_t x_stride, float* y,
+                                                            uint64_t y_stride, int n, int act) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, e = lane & 3;
+    const int m = (blockIdx.x * 4 + wave) * P, r = blockIdx.y * 16 + (lane >> 2);
+    if (m >= n) return;
+    const float* xr[P];
+#pragma unroll
+    for (int j = 0; j < P; j++) xr[j] = x + (uint64_t)min(m + j, n - 1) * x_stride + 4 * e;
+    const float* wr = w + (uint64_t)min(r, rows - 1) * cols + 4 * e;
+    float4 xv[2][P][U], wv[2][U];
+    auto load = [&](int k0, float4 (&xx)[P][U], float4 (&ww)[U]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = min(k0 + 16 * u + 4 * e, cols - 4) - 4 * e;
+            ww[u] = *(const float4*)(wr + k);
+#pragma unroll
+            for (int j = 0; j < P; j++) xx[j][u] = *(const float4*)(xr[j] + k);
+        }
+    };
+    float acc[P] = {};
+    auto run = [&](int k0, const float4 (&xx)[P][U], const float4 (&ww)[U], auto TAIL) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (decltype(TAIL)::value && k0 + 16 * u >= cols) break;
+            float p[P][4];
+            const bool live = !decltype(TAIL)::value || k0 + 16 * u + 4 * e < cols;
+#pragma unroll
+            for (int j = 0; j < P; j++) {
+                p[j][0] = live ? ww[u].x * xx[j][u].x : 0.0f; p[j][1] = live ? ww[u].y * xx[j][u].y : 0.0f;
+                p[j][2] = live ? ww[u].z * xx[j][u].z : 0.0f; p[j][3] = live ? ww[u].w * xx[j][u].w : 0.0f;
+            }
+            static_for<0, 16>([&](auto I) {
+                constexpr int i = decltype(I)::value;
+#pragma unroll
+                for (int j = 0; j < P; j++) acc[j] += quad_bcast<(i >> 2)>(p[j][i & 3]);
+            });
+        }
+    };
+    constexpr int KP = 16 * U;
+    load(0, xv[0], wv[0]);
+    int k0 = 0;
+    for (; k0 + 2 * KP <= cols; k0 += 2 * KP) {
+        load(k0 + KP, xv[1], wv[1]);
+        run(k0, xv[0], wv[0], std::false_type{});
+        load(k0 + 2 * KP, xv[0], wv[0]);
+        run(k0 + KP, xv[1], wv[1], std::false_type{});
+    }
+    for (; k0 < cols; k0 += KP) {
+        run(k0, xv[0], wv[0], std::true_type{});
+        load(k0 + KP, xv[0], wv[0]);
+    }
+    if (e == 0 && r < rows) {
+#pragma unroll
+        for (int j = 0; j < P; j++)
+            if (m + j < n) {
+                float* yo = y + (uint64_t)(m + j) * y_stride + r;
+                *yo = act == 0 ? acc[j] : act == 1 ? silu_f32(*yo) * acc[j] : *yo + acc[j];
+            }
+    }
+}
+template <int RW>
+static void gemm_f32_t(const float* w, int rows, int cols, const float* x, uint64_t x_stride, float* y, uint64_t y_stride,
+                       int n, int act, hipStream_t s) {
+    const dim3 grid((unsigned)((n + GF_M - 1) / GF_M), (unsigned)((rows + 4 * RW - 1) / (4 * RW)));
+    gemm_f32_kernel<RW><<<grid, dim3(256), 0, s>>>(w, rows, cols, x, x_stride, y, y_stride, n, act);
+}
+
 hipError_t launch_gemm_f32(const float* w, int rows, int cols, const float* x, uint64_t x_stride, float* y,
                            uint64_t y_stride, int n, int act, hipStream_t s) {
     if (!rows || !n) return hipSuccess;
-    gemm_f32_kernel<<<dim3((unsigned)((n + GF_M - 1) / GF_M), (unsigned)((rows + GF_R - 1) / GF_R)), dim3(256), 0, s>>>(
-        w, rows, cols, x, x_stride, y, y_stride, n, act);
+    // by outputs (128 rows of 2048 columns, us; quad / RW 1 / 2 / 4): 256 positions 18 / 29 / 41 / 60, 512 28 / 29 / 41 /
+    // 61, 1024 51 / 31 / 41 / 61, 1501 73 / 39 / 45 / 61, 2048 96 / 56 / 46 / 61, 4096 186 / 93 / 89 / 68
+    // (the ring's loads into LDS take 16-byte aligned weight rows, the quad form any float's address)
+    const long long outs = (long long)n * rows;
+    if (outs <= 65536 || (uintptr_t)w % 16) {
+        constexpr int P = 2, U = 8;
+        const dim3 grid((unsigned)((n + 4 * P - 1) / (4 * P)), (unsigned)((rows + 15) / 16));
+        gemm_f32_quad_kernel<P, U><<<grid, dim3(256), 0, s>>>(w, rows, cols, x, x_stride, y, y_stride, n, act);
+    } else if (outs <= 196608) {
+        gemm_f32_t<1>(w, rows, cols, x, x_stride, y, y_stride, n, act, s);
+    } else if (outs <= 262144) {
+        gemm_f32_t<2>(w, rows, cols, x, x_stride, y, y_stride, n, act, s);
+    } else {
+        gemm_f32_t<4>(w, rows, cols, x, x_stride, y, y_stride, n, act, s);
+    }
     return hipGetLastError();
 }
 

@@ -201,14 +201,4 @@ __device__ __forceinline__ float silu_dev(float v) {
 }
 
 
-// f(std::integral_constant<int, I>) for I = B .. E - 1: the index is a constant expression in the body, so register
-// arrays indexed by it stay in registers.
-template <int B, int E, typename Fn>
-__device__ __forceinline__ void static_for(Fn&& f) {
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        static_for<B + 1, E>(f);
-    }
-}
-
 }  // namespace strata

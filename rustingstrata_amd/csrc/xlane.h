@@ -21,6 +21,12 @@ __device__ __forceinline__ int xl32(int v) {
 template <int STEP>
 __device__ __forceinline__ float xl32f(float v) { return __int_as_float(xl32<STEP>(__float_as_int(v))); }
 
+// Lane Q's value of each group of 4 lanes, to all 4 of them (a quad permute; folds into an add that reads it).
+template <int Q>
+__device__ __forceinline__ float quad_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x55 * Q, 0xF, 0xF, true));
+}
+
 // Sum over the 64 lanes of a wave by an xor butterfly (distances 32, 16, .., 1), the same in every lane.
 __device__ __forceinline__ float wave_sum_xor(float v) {
 #pragma unroll
