@@ -638,6 +638,7 @@ static hipError_t gemm_q8_0(const GemmLaunch& g, hipStream_t s) {
 uint64_t gemm_block_positions() { return GM; }
 
 hipError_t launch_gemm(const GemmLaunch& g, hipStream_t s) {
+    if (gemm_few_takes(g)) return launch_gemm_few(g, s);
     if (g.small && g.tiles && g.ty != Q8_0) return launch_gemm_small(g, s);
     switch (g.ty) {
     case Q8_0: return gemm_q8_0(g, s);

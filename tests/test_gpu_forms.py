@@ -4,8 +4,10 @@ import numpy as np
 import pytest
 
 import rustingstrata_amd as S
+from oracle import oracle as O
+from rustingstrata_amd import ggml
 from rustingstrata_amd.backend import F32_TYPE
-from tests.helpers import normal
+from tests.helpers import normal, random_blocks, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +33,54 @@ def test_f32_gemm_forms_are_the_sequential_sum(hip, n, rows, cols, off):
         want += x[:, k:k + 1] * w[None, :, k]
     got = hip.get(yb, np.float32, n * rows).reshape(n, rows)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+# dense GEMMs by items of 16 rows x 16 positions: a block each up to 1280, a wave each up to 2048, the 256-position
+# blocks beyond; rows and positions that do not fill a unit, 1 to 17 super-blocks (terms of 8 at a time)
+@pytest.mark.parametrize("ty", [ggml.Q2_K, ggml.Q3_K, ggml.Q4_K, ggml.Q5_K, ggml.Q6_K, ggml.IQ2_XXS, ggml.IQ3_S, ggml.IQ4_XS])
+@pytest.mark.parametrize("n,rows,cols", [(1, 1, 256), (17, 33, 2304), (40, 130, 4352), (64, 5120, 256), (65, 4097, 512),
+                                         (33, 10912, 256), (33, 10913, 256)])
+def test_dense_gemm_few_positions(hip, ty, n, rows, cols):
+    """gemm_dense against the CPU dots (bit-equal; IQ4_XS sums in float on the CPU: within 1e-5 rel-L2), store and add."""
+    w, x = random_blocks(ty, rows, cols, seed=ty + n), normal((n, cols), seed=rows)
+    t, xb, yb = hip.upload_tensor(ty, w), up(hip, x), hip.alloc(n * rows * 4)
+    hip.gemm_dense(t, n, xb, cols, yb, rows, S.ACT_STORE)
+    got = hip.get(yb, np.float32, n * rows).reshape(n, rows)
+    for m in sorted({0, n // 2, n - 1}):
+        want = O.matvec(ty, w, rows, cols, x[m])
+        if ty == ggml.IQ4_XS:
+            assert rel_l2(got[m], want) <= 1e-5
+        else:
+            assert np.array_equal(got[m].view(np.uint32), want.view(np.uint32)), m
+    hip.gemm_dense(t, n, xb, cols, yb, rows, S.ACT_ADD)
+    assert np.array_equal(hip.get(yb, np.float32, n * rows).reshape(n, rows), got + got)
+
+
+# tile lists of few positions: gathered gate/up and down rows on both sides of the dispatch lines of each kind of type
+@pytest.mark.parametrize("ty", [ggml.Q2_K, ggml.Q5_K, ggml.Q6_K, ggml.IQ4_XS])
+@pytest.mark.parametrize("t,cols", [(3, 512), (32, 2048), (33, 2048), (128, 1536), (129, 256)])
+def test_grouped_gemm_few_positions(hip, ty, t, cols):
+    """The 64-position tile list's GEMMs (SMALL_TILES) give the bits of the plain forms over the same tiles: the
+    paired gate/up, a gathered store, and the rows of X in order (as a down GEMM reads them)."""
+    E, k, rows = 8, 2, 64
+    x, st = normal((t, cols), seed=t), ggml.row_bytes(ty, cols) * rows
+    w = up(hip, random_blocks(ty, 2 * E * rows, cols, seed=ty))
+    ids = up(hip, np.stack([np.random.default_rng(m).choice([0, 1, 2, 5, 7], k, replace=False) for m in range(t)]).astype(np.int32))
+    mt = t * k // 64 + E
+    off, xrow, inv, ntd, tiles = (hip.alloc(b) for b in (4 * (E + 1), 4 * t * k, 4 * t * k, 4, 16 * mt))
+    hip.moe_sort(ids, t, k, E, off, xrow, inv, [(int(w), st)], tiles, mt, ntd, chunk=64)
+    xb, y = up(hip, x), hip.alloc(t * k * rows * 4)
+    xs = up(hip, np.repeat(x, k, axis=0))
+    res = {}
+    for flag in (0, S.SMALL_TILES):
+        out = []
+        hip.gemm_grouped_gate_up(ty, rows, cols, tiles, mt, ntd, xb, cols, t, xrow, y, rows, E * st, flags=flag)
+        out.append(hip.get(y, np.uint32, t * k * rows))
+        for act in (S.ACT_STORE, S.ACT_SWIGLU, S.ACT_ADD):
+            hip.gemm_grouped(ty, rows, cols, tiles, mt, ntd, xb, cols, t, xrow, y, rows, act | flag)
+            out.append(hip.get(y, np.uint32, t * k * rows))
+        hip.gemm_grouped(ty, rows, cols, tiles, mt, ntd, xs, cols, t * k, 0, y, rows, S.ACT_STORE | flag)
+        out.append(hip.get(y, np.uint32, t * k * rows))
+        res[flag] = out
+    for i, (a, b) in enumerate(zip(res[0], res[S.SMALL_TILES])):
+        assert np.array_equal(a, b), i
