@@ -35,6 +35,10 @@ hipError_t launch_gemm(const GemmLaunch& g, hipStream_t s);
 // The form for few positions (gemm_few.hip): whether a GEMM takes it, and its launch.
 bool gemm_few_takes(const GemmLaunch& g);
 hipError_t launch_gemm_few(const GemmLaunch& g, hipStream_t s);
+// A GEMV of several pre-quantized inputs (one matrix, Q8_K numerics) through that form: the same bits;
+// hipErrorNotSupported where it does not apply.
+struct GemvLaunch;
+hipError_t launch_gemv_few(const GemvLaunch& g, hipStream_t s);
 hipError_t launch_gemm_small(const GemmLaunch& g, hipStream_t s);
 // Positions of one GEMM block (a tile list's chunks of this size give every block a full tile).
 uint64_t gemm_block_positions();

@@ -33,7 +33,8 @@ constexpr int FPP = FPM + 4;  // floats of a term row (16-byte pad: rows start i
 // Dense, by items (16 rows x 16 positions; gemm_kernel needs a 128-row block's whole super-block chain whatever the
 // items): Q6_K 5120 x 2048: 5 positions 28.4 -> 7.2, 24 29.6 -> 9.9, 64 (1280 items) 32.1 -> 15.0, 256 (5120) 32.4 ->
 // 36.7; Q4_K 5120 x 2048: 64 27.8 -> 15.7, 100 (2240) 27.8 -> 23.9, 200 28.4 -> 42.7; 2048 x 2048, 256 positions
-// (2048): Q6_K 31.8 -> 16.2, Q4_K 27.8 -> 20.5. A block an item up to 1280 items: 64 positions of 5120 x 2048 15.0
+// (2048): Q6_K 31.8 -> 16.2, Q4_K 27.8 -> 20.5. One unit of positions, whatever the rows: 151936 x 2048, 16 positions
+// (9496): Q6_K 128 -> 69, Q4_K 95 -> 92, Q2_K 82 -> 54 (32 positions: 134 -> 128, 103 -> 179, 87 -> 103). A block an item up to 1280 items: 64 positions of 5120 x 2048 15.0
 // against 16.1 a wave an item (Q4_K 15.7 / 20.1), 256 of 2048 x 2048 22.2 / 16.2 (23.2 / 20.5).
 constexpr long long FEW_DENSE_BLOCK_ITEMS = 1280, FEW_DENSE_ITEMS = 2048;
 long long few_dense_items(int rows, int n) { return (long long)((rows + 15) / 16) * ((n + FPM - 1) / FPM); }
@@ -354,9 +355,22 @@ static hipError_t few_t(const GemmLaunch& g, hipStream_t s) {
     return ksp ? few_launch<T, true>(a, s) : few_launch<T, false>(a, s);
 }
 
+hipError_t launch_gemv_few(const GemvLaunch& g, hipStream_t s) {
+    if (g.ty == Q8_0 || g.numerics != STRATA_NUM_Q8K || !g.xq || g.ids || g.pair || g.cols % 256 ||
+        (uint64_t)g.rows * row_bytes(g.ty, g.cols) >= (1ull << 32) || g.rows > (1 << 24) ||
+        row_bytes(g.ty, g.cols) >= (1u << 24))
+        return hipErrorNotSupported;
+    GemmLaunch m;
+    m.ty = g.ty; m.rows = g.rows; m.cols = g.cols;
+    m.dense_w = g.w; m.dense_n = g.nt; m.n_tiles = 1;
+    m.xq = (const uint8_t*)g.xq; m.n_x = g.n_xrows;
+    m.y = g.y; m.y_stride = g.y_stride; m.act = STRATA_ACT_STORE;
+    return launch_gemm_few(m, s);
+}
+
 bool gemm_few_takes(const GemmLaunch& g) {
     if (g.ty == Q8_0) return false;
-    if (!g.tiles) return few_dense_items(g.rows, g.dense_n) <= FEW_DENSE_ITEMS;
+    if (!g.tiles) return g.dense_n <= FPM || few_dense_items(g.rows, g.dense_n) <= FEW_DENSE_ITEMS;
     if (!g.small) return false;
     const bool sa = g.ty == Q4_K || g.ty == Q5_K || g.ty == IQ4_XS || g.ty == IQ3_S;
     if (g.xrow) return g.n_x <= (sa ? 32 : 128);

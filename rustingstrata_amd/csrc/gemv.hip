@@ -10,6 +10,7 @@
 #include <algorithm>
 
 #include "sbdot.h"
+#include "gemm.h"
 #include "kernels.h"
 #include "xlane.h"
 #include "route.h"
@@ -43,6 +44,7 @@ struct GemvArgs {
     uint32_t ntr_m, ns_m; // magic multipliers and shifts dividing by ntr and nslots (fdiv)
     int ntr_s, ns_s;
     int small;           // single-input kernel, one plain matrix: every tile spans at most GEMV1_CH_SMALL chunks a thread
+    int gxb, gxd, gxs;   // gemv_kernel: bytes, scales and sums of x per super-block in LDS
     int quarter;         // single-input kernel: every tile fits one pass of a wave (at most 64 / G rows), and the four
                          // waves each take one quarter of every super-block (sb_quarter / sb_close)
     // single-input moe kernel that routes its one token first (MODE bit 3): every block ranks the rn logits at rp
@@ -67,8 +69,10 @@ struct GemvArgs {
     int nck;
 };
 
-// LDS layout: [IqTables (IQ types)][x int8: nt * cols][x scales: nt * cols / 32 f32][x sums: nt * cols / 16
-// int32][weight tile], each section rounded up to 16 bytes.
+// LDS layout of gemv_kernel: [IqTables (IQ types)][x int8][x scales, f32][x sums, int32][weight tile], each section
+// rounded up to 16 bytes. Every 256-value super-block of x takes gxb bytes, gxd scales and gxs sums, one 16-byte chunk or
+// word more than its values where the LDS has room: the lanes of a wave read different super-blocks at once, which
+// without the padding all lie in the same banks (151936 x 2048 Q8_0, 3 inputs: 138 -> 100 us).
 __host__ __device__ constexpr uint32_t up16(uint32_t v) { return (v + 15) & ~15u; }
 
 // Sum over the g lanes of each aligned lane group (g a power of two <= 64).
@@ -130,12 +134,13 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
     uint8_t* p = smem;
     IqTables* tab = (IqTables*)p;
     if constexpr (IQ) { load_iq_tables(tab); p += up16(sizeof(IqTables)); }
+    const int nsb = (cols + 255) >> 8;
     int8_t* sx = (int8_t*)p;
-    p += up16(NT * cols);
+    p += up16(NT * nsb * a.gxb);
     float* sd = (float*)p;
-    p += up16(NT * (cols / 32) * 4);
+    p += up16(NT * nsb * a.gxd * 4);
     int* ss = (int*)p;
-    p += up16(NT * (cols / 16) * 4);
+    p += up16(NT * nsb * a.gxs * 4);
     uint8_t* tile = p;
 
     // Tiles: t -> (z, slot, row tile); block b takes tiles b, b + grid, ... and prefetches the next one into
@@ -185,7 +190,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
     issue(sp);
     int cur_xrow = -1;
     const int G = a.G, wave = tid >> 6, lane = tid & 63, gl = lane & (G - 1);
-    const int RPW = 64 / G, nsb = (cols + 255) >> 8;
+    const int RPW = 64 / G;
     while (true) {
         __syncthreads();  // the previous tile's readers are done with the LDS tile (and x)
         if (sp.xrow != cur_xrow) {
@@ -193,12 +198,12 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
             for (int c = tid; c < NT * cols / 16; c += GEMV_THREADS) {
                 const int u = c / (cols / 16), j = c % (cols / 16);
                 const v4u q = *gptr<v4u>((uint64_t)(a.xq + (uint64_t)(sp.xrow + u) * cols + 16 * j));
-                *(v4u*)(sx + 16 * c) = q;
-                ss[c] = sdot4((int)q.x, 0x01010101, sdot4((int)q.y, 0x01010101, sdot4((int)q.z, 0x01010101, sdot4((int)q.w, 0x01010101, 0))));
+                *(v4u*)(sx + (u * nsb + (j >> 4)) * a.gxb + 16 * (j & 15)) = q;
+                ss[(u * nsb + (j >> 4)) * a.gxs + (j & 15)] = sdot4((int)q.x, 0x01010101, sdot4((int)q.y, 0x01010101, sdot4((int)q.z, 0x01010101, sdot4((int)q.w, 0x01010101, 0))));
             }
             for (int c = tid; c < NT * cols / 32; c += GEMV_THREADS) {
                 const int u = c / (cols / 32), j = c % (cols / 32);
-                sd[c] = *gptr<float>((uint64_t)(a.xd + (uint64_t)(sp.xrow + u) * (cols / 32) + j));
+                sd[(u * nsb + (j >> 3)) * a.gxd + (j & 7)] = *gptr<float>((uint64_t)(a.xd + (uint64_t)(sp.xrow + u) * (cols / 32) + j));
             }
             cur_xrow = sp.xrow;
         }
@@ -231,7 +236,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
                     const uint8_t* rowp = tile + (cs.beg - cs.g0) + (uint64_t)rr * a.rb;
 #pragma unroll
                     for (int u = 0; u < NT; u++) {
-                        const XLds xv{sx + u * cols + 256 * sb, sd + u * (cols / 32) + 8 * sb, ss + u * (cols / 16) + 16 * sb};
+                        const XLds xv{sx + (u * nsb + sb) * a.gxb, sd + (u * nsb + sb) * a.gxd, ss + (u * nsb + sb) * a.gxs};
                         const int nv = min(256, cols - 256 * sb);
                         f[u] = Q32 ? sb_dot_q32<T>(rowp + sb * SBB, xv, tab, nv) : sb_dot_q8k<T>(rowp + sb * SBB, xv, tab, nv);
                     }
@@ -857,6 +862,14 @@ static hipError_t gemv_t(const GemvArgs& a, long long grid, size_t smem, hipStre
 }
 
 hipError_t launch_gemv(const GemvLaunch& g, hipStream_t s) {
+    // Several inputs, or one of more columns than the register kernel takes: the MFMA form for few positions decodes a
+    // weight once for all of them (151936 x 2048, 3 inputs, us: Q6_K 121 -> 62, Q4_K 75 -> 43, Q2_K 75 -> 31, IQ4_XS 76 ->
+    // 44; 2048 x 2048: Q6_K 11.8 -> 5.4, Q4_K 8.6 -> 4.6; 2 inputs of 4096 x 14336: Q6_K 48 -> 21). Q8_0, per-32
+    // numerics, paired and routed forms stay here.
+    if (g.nt > 1 || (g.cols > GEMV1_MAX_COLS && g.xq)) {
+        const hipError_t e = launch_gemv_few(g, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     GemvArgs a{};
     a.w = g.w; a.w2 = g.pair ? g.w2 : 0; a.y = g.y; a.y2 = g.pair ? g.y2 : 0;
     a.xq = g.xq; a.xd = g.xq ? (const float*)(g.xq + (uint64_t)g.n_xrows * g.cols) : nullptr;
@@ -937,8 +950,14 @@ hipError_t launch_gemv(const GemvLaunch& g, hipStream_t s) {
         }
         return hipErrorInvalidValue;
     }
-    size_t smem = (iq ? up16(sizeof(IqTables)) : 0) + up16(g.nt * g.cols) + up16(g.nt * (g.cols / 32) * 4) +
-                  up16(g.nt * (g.cols / 16) * 4) + GEMV_TILE + 16;
+    const uint32_t nsb = (uint32_t)(g.cols + 255) / 256;
+    auto lds = [&](int pad) {
+        a.gxb = 256 + 16 * pad; a.gxd = 8 + pad; a.gxs = 16 + pad;
+        return (size_t)(iq ? up16(sizeof(IqTables)) : 0) + up16(g.nt * nsb * a.gxb) + up16(g.nt * nsb * a.gxd * 4) +
+               up16(g.nt * nsb * a.gxs * 4) + GEMV_TILE + 16;
+    };
+    size_t smem = lds(1);
+    if (smem > 160 * 1024) smem = lds(0);
     switch (g.ty) {
     case Q8_0: return gemv_t<Q8_0>(a, grid, smem, s);
     case Q2_K: return gemv_t<Q2_K>(a, grid, smem, s);

@@ -84,3 +84,35 @@ def test_grouped_gemm_few_positions(hip, ty, t, cols):
         res[flag] = out
     for i, (a, b) in enumerate(zip(res[0], res[S.SMALL_TILES])):
         assert np.array_equal(a, b), i
+
+
+@pytest.mark.parametrize("ty", ggml.TYPES)
+@pytest.mark.parametrize("rows,cols", [(3, 256), (33, 2304), (4097, 512), (20500, 256), (40, 20480)])
+def test_gemvn_few_positions_is_gemv(hip, ty, rows, cols):
+    """2 to 4 inputs (and two matrices, gemvq2) give gemv's bits per input, under both numerics, whatever form takes
+    them; rows over the 16384 columns of the register kernel against the CPU dots."""
+    if ggml.row_bytes(ty, cols) > 24512:
+        pytest.skip("row exceeds the GEMV tile")
+    w, x = random_blocks(ty, rows, cols, seed=ty), normal((4, cols), seed=rows)
+    t, xb, y, y2 = hip.upload_tensor(ty, w), up(hip, x), hip.alloc(4 * rows * 4), hip.alloc(4 * rows * 4)
+    y1 = hip.alloc(rows * 4)
+    try:
+        for numerics in (S.NUM_Q8K, S.NUM_Q8_32):
+            hip.set_numerics(numerics)
+            one = []
+            for m in range(4):
+                hip.gemv(t, int(xb) + 4 * m * cols, y1)
+                one.append(hip.get(y1, np.uint32, rows))
+            if numerics == S.NUM_Q8K:
+                assert rel_l2(one[0].view(np.float32), O.matvec(ty, w, rows, cols, x[0])) <= 1e-5
+            for nt in (2, 3, 4):
+                hip.gemvn(t, xb, cols, y, rows, nt)
+                got = hip.get(y, np.uint32, nt * rows).reshape(nt, rows)
+                assert all(np.array_equal(got[m], one[m]) for m in range(nt)), (numerics, nt)
+                if cols <= 16384:
+                    hip.gemvq2(t, t, xb, cols, 0, y, y2, nt)
+                    for yy in (y, y2):
+                        got = hip.get(yy, np.uint32, nt * rows).reshape(nt, rows)
+                        assert all(np.array_equal(got[m], one[m]) for m in range(nt)), (numerics, nt)
+    finally:
+        hip.set_numerics(S.NUM_Q8K)
