@@ -497,22 +497,32 @@ static hipError_t gemm_t(const GemmLaunch& g, hipStream_t s) {
 
 
 // ---- Q8_0 (src/cuda/kernels.cu:380-388): blocks of 32 int8 values, each with its own f16 scale ----
-// The block scales are floats that differ within a super-block, so they cannot fold into integer planes; instead one
-// K=64 MFMA step yields the two blocks' int32 sums separately (lanes 0-31 of the weight operand carry the first
-// block's values and zeros for the second, lanes 32-63 the reverse: two MFMAs per step, no extra MFMA work), and each
-// block closes in float at once: acc += dx (d0 s0 + d1 s1). A block of 4 waves takes a 64-row block of one tile and
-// walks the tile's positions Q8_POS (128) at a time, the next step's X, scales and weights loaded into registers while the current one is computed; wave w owns rows 16 w .. 16 w + 15.
-constexpr int Q8_ROWS = 64, Q8_POS = 128, Q8_SB = 272, Q8_RP = 280;  // rows, positions per pass, bytes per 256 values, LDS row pitch
-constexpr int Q8_NT = Q8_POS / 16;  // MFMA position tiles per pass
+// The block scales are floats that differ within a super-block, so they cannot fold into integer planes: one K=32 MFMA
+// (v_mfma_i32_16x16x32_i8) yields a block's int32 sums, and each closes in float at once, acc += (d dx) s, four VALU
+// instructions an output and block in the CPU's order. Those bound the kernel (4096 x 2048 x 2048: 33K instructions a
+// SIMD, 62 us at 2.1 GHz, against 16 us of MFMAs), so it is built to keep three blocks a CU (three waves a SIMD that
+// share no barrier) at work: a block of 4 waves takes 64 rows x 64 positions, wave w rows 16 w .. 16 w + 15; X rows come
+// by direct global-to-LDS loads one 256-value step ahead (two buffers), raw weight rows into the wave's own LDS region
+// as soon as its current ones are decoded. 4096 x 2048 x 2048: 85 us (172 with 64 x 128 blocks whose loads went
+// through registers, two barriers a step and two half-empty K=64 MFMAs a pair of blocks).
+constexpr int Q8_ROWS = 64, Q8_POS = 64, Q8_SB = 272, Q8_NT = Q8_POS / 16;
+constexpr int Q8_NCH = 19;            // 16-byte chunks of a raw row's LDS pitch: 18 cover 272 bytes at any 2-byte offset, odd
+constexpr int Q8_RP = 16 * Q8_NCH;
+constexpr int Q8_XI = Q8_POS * 16 / 256, Q8_WI = (16 * Q8_NCH + 63) / 64;
 
-__global__ __launch_bounds__(256) void gemm_q8_0_kernel(GemmArgs a) {
-    __shared__ __align__(16) int8_t xs8[Q8_POS * 256];
-    __shared__ __align__(16) uint8_t ws8[Q8_ROWS * Q8_RP];
-    __shared__ float dx8[Q8_POS];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, kl = lane >> 4, aswz = lane & 15;
+__global__ __launch_bounds__(256, 3) void gemm_q8_0_kernel(GemmArgs a) {
+    __shared__ __align__(16) int8_t xs[2][Q8_POS * 256];
+    __shared__ __align__(16) uint8_t ws[Q8_ROWS * Q8_RP];
+    __shared__ __align__(16) float dxs[2][Q8_POS];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, kl = lane >> 4, l16 = lane & 15;
     const int ntiles = a.n_tiles_dev ? min(sload(a.n_tiles_dev), a.max_tiles) : a.max_tiles;
-    const int tile = blockIdx.y, n0 = blockIdx.x * Q8_ROWS;
-    if (tile >= ntiles) return;
+    // XCD x (block ids go round the 8 XCDs) takes a contiguous run of (row block, tile) items, row block major: its few
+    // row blocks' weights stay in its L2 while X streams by
+    const int nrb = (a.rows + Q8_ROWS - 1) / Q8_ROWS;
+    const long long total = (long long)nrb * ntiles, per = (total + NXCD - 1) / NXCD;
+    const long long id = (long long)(blockIdx.x % NXCD) * per + blockIdx.x / NXCD;
+    if ((long long)(blockIdx.x / NXCD) >= per || id >= total) return;
+    const int rb = (int)(id / ntiles), tile = (int)(id - (long long)rb * ntiles), n0 = rb * Q8_ROWS;
     uint64_t w;
     int m0, cnt;
     if (a.tiles) {
@@ -522,88 +532,92 @@ __global__ __launch_bounds__(256) void gemm_q8_0_kernel(GemmArgs a) {
         cnt = min(GM, (int)(t1 >> 32));
     } else {
         w = (uint64_t)a.dense_w;
-        m0 = GM * tile;
-        cnt = min(GM, a.dense_n - m0);
+        m0 = Q8_POS * tile;
+        cnt = min(Q8_POS, a.dense_n - m0);
     }
-    const int cols = a.cols, nsb = cols / 256, rl = 16 * wave + (lane & 15);
-    auto xrow_of = [&](int p) { p = p < cnt ? p : 0; return a.xrow ? a.xrow[m0 + p] : m0 + p; };
-    // Per step (256 values): the X rows of the pass's positions (thread: 4 16-byte chunks), their scales and the
-    // rows' 272 bytes of weights (thread: QW words of the rows' 4-byte-aligned covers) go through registers, the next
-    // step's loads in flight while this one is computed from LDS.
-    constexpr int QW = (Q8_ROWS * (Q8_RP / 4) + 255) / 256;
-    v4i xv[Q8_POS * 16 / 256];
-    uint32_t wv[QW];
-    float dxv = 0.0f;
+    const int cols = a.cols, nsb = cols / 256, rl = 16 * wave + l16;
+    uint8_t* raw = ws + 16 * Q8_RP * wave;
+    // weight instruction i: chunk c = 64 i + lane of the wave's 16 rows, chunk c % NCH of row c / NCH
+    uint32_t wo[Q8_WI];
+    bool wl[Q8_WI];
+#pragma unroll
+    for (int i = 0; i < Q8_WI; i++) {
+        const int c = 64 * i + lane, r = c / Q8_NCH;
+        const uint32_t t = (uint32_t)(w & 15) + __umul24((uint32_t)min(n0 + 16 * wave + min(r, 15), a.rows - 1), (uint32_t)a.rb);
+        wo[i] = (t & ~15u) + 16 * (uint32_t)(c - r * Q8_NCH);
+        wl[i] = r < 16 && wo[i] < t + Q8_SB;
+    }
+    auto load_w = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < Q8_WI; i++)
+            if (wl[i]) load_lds16_so((w & ~(uint64_t)15) + (uint64_t)s * Q8_SB, wo[i], raw + 16 * 64 * i);
+    };
+    // this lane's raw row (272 bytes a super-block: the byte offset in its cover is the same for all of them)
+    const uint8_t* b = raw + l16 * Q8_RP + (((uint32_t)(w & 15) + __umul24((uint32_t)min(n0 + rl, a.rows - 1), (uint32_t)a.rb)) & 15);
     for (int p0 = 0; p0 < cnt; p0 += Q8_POS) {
-        uint32_t xoff[Q8_POS * 16 / 256];
+        const int pc = min(Q8_POS, cnt - p0);  // positions of this pass; those past it read its first row
+        auto xrow_of = [&](int p) { p = m0 + p0 + (p < pc ? p : 0); return a.xrow ? a.xrow[p] : p; };
+        // X instruction j of a wave: positions 4 (XI wave + j) + lane / 16, LDS chunk lane % 16 holding X chunk
+        // (lane % 16) ^ (p & 15)
+        uint32_t xo[Q8_XI];
 #pragma unroll
-        for (int u = 0; u < Q8_POS * 16 / 256; u++) {
-            const int c = tid + 256 * u, p = c >> 4, ch = c & 15;
-            xoff[u] = (uint32_t)xrow_of(p0 + p) * (uint32_t)cols + 16 * ch;
+        for (int j = 0; j < Q8_XI; j++) {
+            const int p = 4 * (Q8_XI * wave + j) + (lane >> 4);
+            xo[j] = (uint32_t)xrow_of(p) * (uint32_t)cols + 16 * ((lane & 15) ^ (p & 15));
         }
-        const uint32_t dxo = (uint32_t)xrow_of(p0 + (tid & (Q8_POS - 1))) * (uint32_t)(cols / 32);
-        auto fetch = [&](int sb) {
+        const uint32_t dxo = 4u * (uint32_t)xrow_of(lane) * (uint32_t)(cols / 32);
+        auto load_x = [&](int s, int buf) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < Q8_POS * 16 / 256; u++) xv[u] = *gptr<v4i>((uint64_t)(a.xq + xoff[u] + 256 * sb));
-            if (tid < Q8_POS) dxv = *gptr<float>((uint64_t)(a.xd + dxo + 8 * sb));
-#pragma unroll
-            for (int u = 0; u < QW; u++) {
-                const int c = tid + 256 * u, r = c / (Q8_RP / 4), j = c % (Q8_RP / 4);
-                const uint64_t beg = w + (uint64_t)min(n0 + min(r, Q8_ROWS - 1), a.rows - 1) * a.rb + (uint64_t)sb * Q8_SB;
-                const uint64_t a4 = beg & ~(uint64_t)3;
-                wv[u] = 0;
-                if (c < Q8_ROWS * (Q8_RP / 4) && a4 + 4 * (uint64_t)j < beg + Q8_SB) wv[u] = *gptr<uint32_t>(a4 + 4 * (uint64_t)j);
-            }
+            for (int j = 0; j < Q8_XI; j++) load_lds16_so((uint64_t)(a.xq + 256 * s), xo[j], xs[buf] + 1024 * (Q8_XI * wave + j));
+            if (wave == 0) load_lds4_so((uint64_t)(a.xd + 8 * s), dxo, dxs[buf]);
         };
         float acc[Q8_NT][4];
 #pragma unroll
         for (int i = 0; i < Q8_NT; i++)
 #pragma unroll
             for (int q = 0; q < 4; q++) acc[i][q] = 0.0f;
-        fetch(0);
-        for (int sb = 0; sb < nsb; sb++) {
-            __syncthreads();  // the previous step's readers are done
-            // X: Q8_POS positions x 256 bytes, 16-byte chunk c of position p at chunk c ^ (p & 15)
+        load_x(0, 0);
+        load_w(0);
+        wait_loads();
+        lds_barrier();
+        for (int s = 0; s < nsb; s++) {
+            const int buf = s & 1;
+            if (s + 1 < nsb) load_x(s + 1, buf ^ 1);
+            // the row's blocks: this lane's 8 values of each (8 kl ..) and its scale
+            uint32_t bq[8][2];
+            float d[8];
 #pragma unroll
-            for (int u = 0; u < Q8_POS * 16 / 256; u++) {
-                const int c = tid + 256 * u, p = c >> 4, ch = c & 15;
-                *(v4i*)(xs8 + p * 256 + 16 * (ch ^ (p & 15))) = xv[u];
+            for (int g = 0; g < 8; g++) {
+                words_a2<2>(b + 34 * g + 2 + 8 * kl, bq[g]);
+                d[g] = h16(b + 34 * g);
             }
-            if (tid < Q8_POS) dx8[tid] = dxv;
+            wait_lds();  // decoded: the raw region takes the next step's rows
+            asm volatile("" : : : "memory");
+            if (s + 1 < nsb) load_w(s + 1);
+            const int8_t* xp = xs[buf] + l16 * 256 + 8 * (kl & 1);
+            static_for<0, Q8_NT>([&](auto I) __attribute__((always_inline)) {
+                constexpr int i = decltype(I)::value;
+                if (16 * i >= pc) return;
+                const float4 dv = *(const float4*)(dxs[buf] + 16 * i + 4 * kl);
+                const float dq[4] = {dv.x, dv.y, dv.z, dv.w};
 #pragma unroll
-            for (int u = 0; u < QW; u++) {
-                const int c = tid + 256 * u;
-                if (c < Q8_ROWS * (Q8_RP / 4)) *(uint32_t*)(ws8 + 4 * c) = wv[u];
-            }
-            __syncthreads();
-            if (sb + 1 < nsb) fetch(sb + 1);
-            const uint64_t rbeg = w + (uint64_t)min(n0 + rl, a.rows - 1) * a.rb + (uint64_t)sb * Q8_SB;
-            const uint8_t* wr = ws8 + rl * Q8_RP + (uint32_t)(rbeg & 3);
+                for (int h = 0; h < 8; h += 4) {  // four blocks at a time: registers
+                    v4i c[4];
 #pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                // this lane's 16 values: block 2 kk + kl / 2, values 16 (kl & 1) ..
-                uint32_t qv[4];
-                words_a2<4>(wr + 34 * (2 * kk + (kl >> 1)) + 2 + 16 * (kl & 1), qv);
-                const v4i qw = {(int)qv[0], (int)qv[1], (int)qv[2], (int)qv[3]}, z = {0, 0, 0, 0};
-                const v4i b0 = kl < 2 ? qw : z, b1 = kl < 2 ? z : qw;
-                const float d0 = h16(wr + 34 * (2 * kk)), d1 = h16(wr + 34 * (2 * kk + 1));
-                // the 2 Q8_NT MFMAs first, then their closes (each result is used 2 Q8_NT issues after its MFMA)
-                v4i c0[Q8_NT], c1[Q8_NT];
-#pragma unroll
-                for (int i = 0; i < Q8_NT; i++) {
-                    const v4i av = *(const v4i*)(xs8 + (16 * i + aswz) * 256 + 16 * ((4 * kk + kl) ^ aswz));
-                    c0[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, b0, z, 0, 0, 0);
-                    c1[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, b1, z, 0, 0, 0);
-                }
-#pragma unroll
-                for (int i = 0; i < Q8_NT; i++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {  // sum += (d dx) s per 32-block, in order (src/cpu_moe.rs:319-325)
-                        const float dxq = dx8[16 * i + 4 * kl + q];
-                        acc[i][q] = acc[i][q] + (d0 * dxq) * (float)c0[i][q];
-                        acc[i][q] = acc[i][q] + (d1 * dxq) * (float)c1[i][q];
+                    for (int g = h; g < h + 4; g++) {
+                        const long av = *(const long*)(xp + 4096 * i + 16 * ((2 * g + (kl >> 1)) ^ l16));
+                        const long bv = (long)(((uint64_t)bq[g][1] << 32) | bq[g][0]);
+                        c[g - h] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv, (v4i){0, 0, 0, 0}, 0, 0, 0);
                     }
-            }
+#pragma unroll
+                    for (int g = h; g < h + 4; g++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++)  // sum += (d dx) s per 32-block, in order (src/cpu_moe.rs:319-325)
+                            acc[i][q] = acc[i][q] + (d[g] * dq[q]) * (float)c[g - h][q];
+                }
+            });
+            wait_loads();
+            lds_barrier();
         }
         // outputs: weight row n0 + rl, positions p0 + 16 i + 4 kl + q
         if (n0 + rl < a.rows) {
@@ -611,9 +625,9 @@ __global__ __launch_bounds__(256) void gemm_q8_0_kernel(GemmArgs a) {
             for (int i = 0; i < Q8_NT; i++)
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    const int m = p0 + 16 * i + 4 * kl + q;
-                    if (m < cnt) {
-                        float* yp = a.y + (int64_t)(m0 + m) * a.y_stride + n0 + rl;
+                    const int m = 16 * i + 4 * kl + q;
+                    if (m < pc) {
+                        float* yp = a.y + (int64_t)(m0 + p0 + m) * a.y_stride + n0 + rl;
                         if (a.act == STRATA_ACT_STORE) *yp = acc[i][q];
                         else if (a.act == STRATA_ACT_SWIGLU) *yp = silu_dev(*yp) * acc[i][q];
                         else *yp += acc[i][q];
@@ -629,9 +643,11 @@ static hipError_t gemm_q8_0(const GemmLaunch& g, hipStream_t s) {
     a.xq = (const int8_t*)g.xq; a.xd = (const float*)(g.xq + (uint64_t)g.n_x * g.cols);
     a.xrow = g.xrow; a.y = g.y; a.y_stride = g.y_stride; a.rows = g.rows; a.cols = g.cols; a.act = g.act;
     a.rb = row_bytes(Q8_0, g.cols);
-    a.max_tiles = g.n_tiles;
-    if (g.n_tiles > 65535) return hipErrorInvalidValue;
-    gemm_q8_0_kernel<<<dim3((unsigned)((g.rows + Q8_ROWS - 1) / Q8_ROWS), (unsigned)g.n_tiles), 256, 0, s>>>(a);
+    a.max_tiles = g.tiles ? g.n_tiles : (g.dense_n + Q8_POS - 1) / Q8_POS;
+    const long long total = (long long)((g.rows + Q8_ROWS - 1) / Q8_ROWS) * a.max_tiles;
+    const long long grid = (total + NXCD - 1) / NXCD * NXCD;
+    if (grid >= (1ll << 31)) return hipErrorInvalidValue;
+    gemm_q8_0_kernel<<<dim3((unsigned)grid), 256, 0, s>>>(a);
     return hipGetLastError();
 }
 

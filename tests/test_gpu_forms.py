@@ -37,8 +37,9 @@ def test_f32_gemm_forms_are_the_sequential_sum(hip, n, rows, cols, off):
 
 # dense GEMMs by items of 16 rows x 16 positions: a block each up to 1280, a wave each up to 2048, the 256-position
 # blocks beyond; rows and positions that do not fill a unit, 1 to 17 super-blocks (terms of 8 at a time)
-@pytest.mark.parametrize("ty", [ggml.Q2_K, ggml.Q3_K, ggml.Q4_K, ggml.Q5_K, ggml.Q6_K, ggml.IQ2_XXS, ggml.IQ3_S, ggml.IQ4_XS])
-@pytest.mark.parametrize("n,rows,cols", [(1, 1, 256), (17, 33, 2304), (40, 130, 4352), (64, 5120, 256), (65, 4097, 512),
+# (Q8_0: blocks of 64 rows x 64 positions)
+@pytest.mark.parametrize("ty", ggml.TYPES)
+@pytest.mark.parametrize("n,rows,cols", [(1, 1, 256), (64, 64, 512), (129, 63, 768), (17, 33, 2304), (40, 130, 4352), (64, 5120, 256), (65, 4097, 512),
                                          (33, 10912, 256), (33, 10913, 256)])
 def test_dense_gemm_few_positions(hip, ty, n, rows, cols):
     """gemm_dense against the CPU dots (bit-equal; IQ4_XS sums in float on the CPU: within 1e-5 rel-L2), store and add."""
