@@ -569,63 +569,85 @@ hipError_t launch_attn_decode(const float* q, const uint16_t* kc, const uint16_t
 }
 
 // ---------------- prefill ----------------
-// grid (ceil(ceil(t / 16) / 2), nkv), G waves: wave w is query head g G + w over the block's two 16-query MFMA columns
-// j, the 16-row tiles qb and ceil(t / 16) - 1 - qb (from the two ends of the chunk, so that the blocks' causal work
-// is even), and every K/V tile in LDS serves the whole GQA group. Query row i sits at position step[0] + i and sees
-// keys base(i) .. step[0] + i (base 0, or the sliding window's start); a column takes part in a key tile only while
-// the tile holds keys its rows see. Per tile of 64 keys:
-//   S^T (16 keys x 16 queries, 4 key sub-tiles kt) = sum over dims of K (A: key row, 8 dims a lane) with Q^T hi and lo
-//   (B: query column, the same 8 dims); lane holds keys 16 kt + 4 (l / 16) + i of query 16 j + l % 16.
-//   Online softmax per query column (the lane's 16 values, then across the 4 lane groups).
-//   O^T (16 dims x 16 queries, 8 dim tiles dt) += V^T (A: dim row, 8 keys) P^T hi and lo (B: the lane's own p values:
-//   keys 4 (l / 16) + i of sub-tiles 2 c and 2 c + 1 make the 8 K-elements of k-step c, and V^T's A fragment reads
-//   the same keys).
+// A block of 4 waves takes HW = min(G, 4) query heads of one KV head x RT = 4 / HW tiles of 32 query rows (a wave each).
+// Blocks run over the head groups first (an XCD keeps few KV heads' K and V in its L2) and the row tiles from the last,
+// longest one, so that the short ones fill the CUs that finish early. Query row i sits at position step[0] + i and sees keys
+// base(i) .. step[0] + i (base 0, or the sliding window's start). Per tile of 64 keys, on v_mfma_f32_32x32x16_f16:
+//   S^T (32 keys x 32 queries, 2 key sub-tiles mt) = sum over dims of K (A: key row, 8 dims a lane) with Q^T hi and lo
+//   (B: query column, the same 8 dims); lane holds keys 32 mt + 8 (i / 4) + 4 (l / 32) + i % 4 of query l % 32.
+//   Online softmax per query column (the lane's 32 values, then the other half-wave's by one lane swap; the sums stay
+//   per lane until the end).
+//   O^T (32 dims x 32 queries) += V^T (A: dim row, 8 keys) P^T hi and lo (B: the lane's own p values: i = 8 u .. 8 u + 7
+//   of sub-tile mt make the 8 K-elements of a k-step, and V^T's A fragment reads the same keys).
+// A wave issues 64 MFMAs of 32 cycles a key tile (2048 cycles: with the hi / lo splits 275 GFLOP for 4096 tokens, 32
+// heads of 128 over 4) and ~270 other VALU instructions, 32 of them quarter-rate exps: the two overlap between the two
+// waves of a SIMD for 54% MFMA time. Measured there 273 us; 381 with 16 x 16 MFMAs (a SIMD issues about two VALU
+// instructions beside an MFMA of 16 cycles, so half the MFMAs leave room for more), a rescale of the accumulators in most
+// tiles, the weights' scale and f16 remainders as instructions of their own and four cross-lane steps a tile. Rows of one
+// tile instead of two from opposite ends keep a sliding window's key range short (window 1024: 545 -> 147 us).
 constexpr int PF_BK = 64;  // keys a tile (PfLayout's 64)
+constexpr int PF_Q = 32, PF_W = 4;  // query rows a wave; waves a block
+typedef float f16v __attribute__((ext_vector_type(16)));
 
-template <int HD, int G>
-__global__ __launch_bounds__(64 * G) void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
-                                                              const uint16_t* __restrict__ vc, const float* __restrict__ qg,
-                                                              float* __restrict__ out, const int* step, int T, int nh,
-                                                              int nkv, float scale, const float* __restrict__ sink,
-                                                              int win) {
+// Eight softmax weights p (at most 8) times PF_SCALE as f16 hi and lo parts for the P V MFMA: hi = f16(p c), lo the exact
+// remainder p c - hi rounded likewise, both to nearest, so hi + lo carries each weight to 2^-22 of its value and the lo
+// parts stay normal f16 numbers for weights down to 2^-14. The mixed-precision multiply-adds scale, round and read the
+// f16 halves in place.
+constexpr float PF_SCALE = 2048.0f;
+__device__ __forceinline__ void split_w8(const float* p, h8& hi, h8& lo) {
+    typedef float f2v __attribute__((ext_vector_type(2)));
+    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+    uint32_t hw[4], lw[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float a = p[2 * e], b = p[2 * e + 1];
+        float ra, rb;
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(hw[e]) : "v"(a), "s"(PF_SCALE));
+        asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(hw[e]) : "v"(b), "s"(PF_SCALE));
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(ra) : "v"(a), "s"(PF_SCALE), "v"(hw[e]));
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(rb) : "v"(b), "s"(PF_SCALE), "v"(hw[e]));
+        lw[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2v){ra, rb}, h2v));
+    }
+    hi = __builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3]));
+    lo = __builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3]));
+}
+// The larger of this lane's value and that of the lane 32 away.
+__device__ __forceinline__ float max_half(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+template <int HD, int HW>
+__global__ __launch_bounds__(64 * PF_W, 2) void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
+                                                                  const uint16_t* __restrict__ vc, const float* __restrict__ qg,
+                                                                  float* __restrict__ out, const int* step, int T, int nh,
+                                                                  int nkv, float scale, const float* __restrict__ sink,
+                                                                  int win) {
     using L = PfLayout<HD>;
-    constexpr int KS = HD / 32, DT = HD / 16, NTH = 64 * G;
+    constexpr int KS = HD / 16, DT = HD / 32, NTH = 64 * PF_W, ND = HD / 8, RT = PF_W / HW;
     __shared__ __align__(16) uint16_t ks[PF_BK * L::KP];
     __shared__ __align__(16) uint16_t vs[HD * L::VP];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
-    const int g = blockIdx.y, h = g * G + wave, pos0 = step[0];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hf = lane >> 5;
+    const int nhg = nh / HW, hg = blockIdx.x % nhg, tb = blockIdx.x / nhg, ntb = gridDim.x / nhg;
+    const int h = hg * HW + wave % HW, g = hg * HW / (nh / nkv), pos0 = step[0];
     const uint64_t kvd = (uint64_t)nkv * HD;
-    // the block's two query columns are 16-row tiles from opposite ends of the T rows (tiles qb and nht - 1 - qb),
-    // so every block has about the same causal work; each column's MFMAs and softmax stop at its own last key
-    const int nht = (T + 15) / 16, qb = blockIdx.x;
-    const int r0[2] = {16 * qb, 16 * (nht - 1 - qb)};
-    const bool two = nht - 1 - qb != qb;
-    int lastj[2], firstj[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        lastj[j] = pos0 + min(r0[j] + 15, T - 1);  // the last key the column's rows see
-        firstj[j] = win > 0 ? max(pos0 + r0[j] + 1 - win, 0) : 0;
-    }
-    if (!two) {
-        lastj[1] = -1;
-        firstj[1] = INT_MAX;
-    }
-    const int last = max(lastj[0], lastj[1]), first = min(firstj[0], firstj[1]);
-    // Q^T fragments (B operand): query r0[j] + l16, dims 32 ks + 8 lg .. + 7, split into f16 hi and lo after scaling
+    const int rb = PF_Q * RT * (ntb - 1 - tb), r0 = rb + PF_Q * (wave / HW), row = r0 + l32;
+    // the keys that the block's rows see, and the wave's (none for a wave past the last row)
+    const int last = pos0 + min(rb + PF_Q * RT - 1, T - 1), first = win > 0 ? max(pos0 + rb + 1 - win, 0) : 0;
+    const int lastw = r0 < T ? pos0 + min(r0 + PF_Q - 1, T - 1) : -1, firstw = win > 0 ? max(pos0 + r0 + 1 - win, 0) : 0;
+    // Q^T fragments (B operand): query row l32, dims 16 k + 8 hf .. + 7, split into f16 hi and lo after scaling
     // the query by a power of two that puts its largest value in [2^13, 2^14): the lo parts then stay normal f16
-    // numbers (no subnormal precision loss) and the hi parts cannot overflow. usc[j] undoes it (times `scale`).
-    h8 qh[2][KS], ql[2][KS];
-    float usc[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int row = r0[j] + l16;
+    // numbers (no subnormal precision loss) and the hi parts cannot overflow. usc undoes it (times `scale`).
+    h8 qh[KS], ql[KS];
+    float usc;
+    {
         const float* qr = q + (uint64_t)row * nh * HD + h * HD;
         float v[KS][8];
         float mx = 0.0f;
 #pragma unroll
         for (int k = 0; k < KS; k++) {
-            if (row < T && (j == 0 || two)) {
-                const float4 a = *(const float4*)(qr + 32 * k + 8 * lg), b = *(const float4*)(qr + 32 * k + 8 * lg + 4);
+            if (row < T) {
+                const float4 a = *(const float4*)(qr + 16 * k + 8 * hf), b = *(const float4*)(qr + 16 * k + 8 * hf + 4);
                 v[k][0] = a.x; v[k][1] = a.y; v[k][2] = a.z; v[k][3] = a.w;
                 v[k][4] = b.x; v[k][5] = b.y; v[k][6] = b.z; v[k][7] = b.w;
             } else {
@@ -635,170 +657,167 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(const float* __res
 #pragma unroll
             for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf(v[k][e]));
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = max_half(mx);
         int ex = 0;
         if (mx > 0.0f) (void)frexpf(mx, &ex);  // mx < 2^ex
         const float up = ldexpf(1.0f, 14 - ex);
-        usc[j] = ldexpf(scale * LOG2E, ex - 14);  // scores in log2 units: the softmax's exps are exp2s
+        usc = ldexpf(scale * LOG2E, ex - 14);  // scores in log2 units: the softmax's exps are exp2s
 #pragma unroll
         for (int k = 0; k < KS; k++)
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const float x = v[k][e] * up;
                 const _Float16 hi = (_Float16)x;
-                qh[j][k][e] = hi;
-                ql[j][k][e] = (_Float16)(x - (float)hi);
+                qh[k][e] = hi;
+                ql[k][e] = (_Float16)(x - (float)hi);
             }
     }
-    f4 o[2][DT];
+    f16v o[DT];
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int d = 0; d < DT; d++)
 #pragma unroll
-        for (int d = 0; d < DT; d++) o[j][d] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
-    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
-    const int qpos[2] = {pos0 + r0[0] + l16, pos0 + r0[1] + l16};  // the lane's query position per column j
-    // K tile [key][dim] and V tile transposed [dim][key], chunk i = tid + NTH u of a tile: key i % 64, dims
-    // 8 (i / 64) ..; the next tile's chunks are loaded into registers while this one is computed. Keys past `last`
-    // are zeros (finite: p = 0 times them).
-    constexpr int NPT = PF_BK * HD / 8 / NTH;  // 16-byte chunks a thread of each of K and V
-    uint4 kr[NPT], vr4[NPT];
-    auto fetch = [&](int k0) {
+        for (int i = 0; i < 16; i++) o[d][i] = 0.0f;
+    // m: a running maximum that may lag by 3, so the weights 2^(s - m) are at most 8; l: this lane's share of their sum
+    float m = -INFINITY, l = 0.0f;
+    const int qpos = pos0 + row;  // the lane's query position
+    // K tile [key][dim] and V tile transposed [dim][key]; K chunk i = tid + NTH u of a tile: key i / ND, dims 8 (i % ND) ..;
+    // V items: keys 2 a, 2 a + 1 and dims 8 c .., packed in pairs of keys, 8 a's x 8 c's a wave (whole 128-byte lines, and
+    // the transposed stores spread over the banks). The next tile's chunks are loaded into
+    // registers while this one is computed. Keys past `last` read its row (finite: p = 0 times them).
+    constexpr int NPK = PF_BK * ND / NTH, NPV = PF_BK / 2 * ND / NTH;
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    v4u kr[NPK], vr[NPV][2];
+    const int kk = tid / ND, kcol = 8 * (tid % ND);                                             // K: key, dim of chunk 0
+    const int vk = 2 * (((tid >> 3) & 7) + 8 * (wave / (ND / 8))), vcol = 8 * ((tid & 7) + 8 * (wave % (ND / 8)));  // V: item 0
+    constexpr int KST = NTH / ND, VST = 16 * PF_W / (ND / 8);                                   // keys to the next chunk / item
+    // a tile's loads: its scalar base + a 32-bit offset of the lane's row in it (24-bit multiply-adds)
+    const uint32_t kvd2 = 2 * (uint32_t)kvd, kc2 = 2 * (g * HD + kcol), vc2 = 2 * (g * HD + vcol);
+    auto fetch = [&](int k0) __attribute__((always_inline)) {
+        const uint64_t kb = (uint64_t)kc + (uint64_t)k0 * kvd2, vb = (uint64_t)vc + (uint64_t)k0 * kvd2;
+        const int lim = last - k0;
 #pragma unroll
-        for (int u = 0; u < NPT; u++) {
-            const int i = tid + NTH * u, key = i % PF_BK, c = (i / PF_BK) * 8, kp = k0 + key;
-            kr[u] = make_uint4(0, 0, 0, 0);
-            vr4[u] = kr[u];
-            if (kp <= last) {
-                kr[u] = *(const uint4*)(kc + (uint64_t)kp * kvd + g * HD + c);
-                vr4[u] = *(const uint4*)(vc + (uint64_t)kp * kvd + g * HD + c);
-            }
-        }
+        for (int u = 0; u < NPK; u++) kr[u] = *gptr<v4u>(kb + (__umul24((uint32_t)min(KST * u + kk, lim), kvd2) + kc2));
+#pragma unroll
+        for (int u = 0; u < NPV; u++)
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                vr[u][e] = *gptr<v4u>(vb + (__umul24((uint32_t)min(VST * u + e + vk, lim), kvd2) + vc2));
     };
     const int kbeg = first / PF_BK * PF_BK;
     fetch(kbeg);
     for (int k0 = kbeg; k0 <= last; k0 += PF_BK) {
         __syncthreads();  // the previous tile's readers are done
 #pragma unroll
-        for (int u = 0; u < NPT; u++) {
-            const int i = tid + NTH * u, key = i % PF_BK, c = (i / PF_BK) * 8;
-            *(uint4*)&ks[key * L::KP + c] = kr[u];
-            const uint32_t w4[4] = {vr4[u].x, vr4[u].y, vr4[u].z, vr4[u].w};
+        for (int u = 0; u < NPK; u++) *(v4u*)&ks[(kk + KST * u) * L::KP + kcol] = kr[u];
 #pragma unroll
-            for (int e = 0; e < 8; e++) vs[(c + e) * L::VP + key] = (uint16_t)(w4[e >> 1] >> (16 * (e & 1)));
-        }
+        for (int u = 0; u < NPV; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t a = vr[u][0][e], b = vr[u][1][e];
+                *(uint32_t*)&vs[(vcol + 2 * e) * L::VP + vk + VST * u] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+                *(uint32_t*)&vs[(vcol + 2 * e + 1) * L::VP + vk + VST * u] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+            }
         __syncthreads();
         if (k0 + PF_BK <= last) fetch(k0 + PF_BK);
-        bool live[2];
-#pragma unroll
-        for (int j = 0; j < 2; j++) live[j] = k0 <= lastj[j] && k0 + PF_BK - 1 >= firstj[j];
+        if (RT > 1 && (k0 > lastw || k0 + PF_BK - 1 < firstw)) continue;
         // S^T
-        f4 s[2][4];
+        f16v s[2];
+        f16v z;
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++) {
-            h8 kf[KS];
+        for (int i = 0; i < 16; i++) z[i] = 0.0f;
 #pragma unroll
-            for (int k = 0; k < KS; k++) kf[k] = *(const h8*)&ks[(16 * kt + l16) * L::KP + 32 * k + 8 * lg];
+        for (int k = 0; k < KS; k++) {  // (the two sub-tiles' chains interleaved)
+            const h8 k0f = *(const h8*)&ks[l32 * L::KP + 16 * k + 8 * hf], k1f = *(const h8*)&ks[(32 + l32) * L::KP + 16 * k + 8 * hf];
+            s[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k0f, qh[k], k ? s[0] : z, 0, 0, 0);
+            s[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k1f, qh[k], k ? s[1] : z, 0, 0, 0);
+            s[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k0f, ql[k], s[0], 0, 0, 0);
+            s[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k1f, ql[k], s[1], 0, 0, 0);
+        }
+        // keys outside first .. qpos masked, on the tiles that have such keys
+        if (k0 + PF_BK - 1 > pos0 + r0 || (win > 0 && k0 < lastw + 1 - win)) {
+            const int lo = win > 0 ? qpos + 1 - win : INT_MIN;
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                f4 c = (f4){0.0f, 0.0f, 0.0f, 0.0f};
-                if (live[j])
+            for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-                for (int k = 0; k < KS; k++) {
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[k], qh[j][k], c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[k], ql[j][k], c, 0, 0, 0);
+                for (int i = 0; i < 16; i++) {
+                    const int kp = k0 + 32 * mt + 8 * (i >> 2) + 4 * hf + (i & 3);
+                    if (kp > qpos || kp < lo) s[mt][i] = -INFINITY;
                 }
-                s[j][kt] = c;
+        }
+        // online softmax of the query column (raw scores: usc (> 0) is applied in the exponent's fma)
+        float mx = -INFINITY;
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[mt][i]);
+        mx = max_half(mx);
+        // m follows the maximum only when a weight of the column would pass 8: the accumulators are rescaled in the first
+        // tiles and hardly ever after them. (Column by column: a row's bits do not depend on the rows beside it, so not on
+        // how a prompt is cut into chunks.)
+        const float mxs = mx * usc;  // (a positive factor keeps the order)
+        if (__ballot(mxs > m + 3.0f)) {
+            const float mnew = mxs > m + 3.0f ? mxs : m, alpha = m == -INFINITY ? 0.0f : exp2_hw(m - mnew);
+            l *= alpha;
+#pragma unroll
+            for (int d = 0; d < DT; d++) o[d] *= alpha;
+            m = mnew;
+        }
+        const float mref = m == -INFINITY ? 0.0f : m;  // a column with no key yet: every p is 0
+        float sum = 0.0f;
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const float p = exp2_hw(__builtin_fmaf(s[mt][i], usc, -mref));  // exp2(-inf) = 0
+                s[mt][i] = p;
+                sum += p;
             }
-        }
-        // online softmax per query column; keys outside first .. qpos masked, on the tiles that have such keys
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            if (!live[j]) continue;
-            const bool edge = k0 + PF_BK - 1 > pos0 + r0[j] || (win > 0 && k0 < lastj[j] + 1 - win);
-            const int qp = qpos[j], lo = win > 0 ? qp + 1 - win : INT_MIN;
-            float mx = -INFINITY;
-#pragma unroll
-            for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int kp = k0 + 16 * kt + 4 * lg + i;
-                    float v = s[j][kt][i];  // the raw score: usc (> 0) is applied in the exponent's fma
-                    if (edge && (kp > qp || kp < lo)) v = -INFINITY;
-                    s[j][kt][i] = v;
-                    mx = fmaxf(mx, v);
-                }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float mnew = fmaxf(m[j], mx * usc[j]);  // max(v) usc = max(v usc): a positive factor keeps the order
-            const float alpha = m[j] == -INFINITY ? 0.0f : exp2_hw(m[j] - mnew);
-            const float mref = mnew == -INFINITY ? 0.0f : mnew;  // a column with no key yet: every p is 0
-            float sum = 0.0f;
-#pragma unroll
-            for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float p = exp2_hw(__builtin_fmaf(s[j][kt][i], usc[j], -mref));  // exp2(-inf) = 0
-                    s[j][kt][i] = p;
-                    sum += p;
-                }
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
-            l[j] = l[j] * alpha + sum;
-            m[j] = mnew;
-            if (__ballot(alpha != 1.0f))  // the running maximum moved for some column of the wave
-#pragma unroll
-                for (int d = 0; d < DT; d++) o[j][d] *= alpha;
-        }
+        l += sum;
         // O^T += V^T P^T
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            h8 ph[2], pl[2];
+        for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                if (!live[j]) continue;
+            for (int u = 0; u < 2; u++) {
                 float p[8];
 #pragma unroll
-                for (int e = 0; e < 8; e++) p[e] = s[j][2 * c + (e >> 2)][e & 3];
-                split_p8(p, ph[j], pl[j]);
-            }
+                for (int e = 0; e < 8; e++) p[e] = s[mt][8 * u + e];
+                h8 ph, pl;
+                split_w8(p, ph, pl);
+                h8 vf[DT];
 #pragma unroll
-            for (int d = 0; d < DT; d++) {
-                const uint16_t* vr = &vs[(16 * d + l16) * L::VP + 32 * c + 4 * lg];
-                const uint2 a0 = *(const uint2*)vr, a1 = *(const uint2*)(vr + 16);
-                const h8 vf = __builtin_bit_cast(h8, make_uint4(a0.x, a0.y, a1.x, a1.y));
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    if (!live[j]) continue;
-                    o[j][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph[j], o[j][d], 0, 0, 0);
-                    o[j][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[j], o[j][d], 0, 0, 0);
+                for (int d = 0; d < DT; d++) {
+                    const uint16_t* vp = &vs[(32 * d + l32) * L::VP + 32 * mt + 16 * u + 4 * hf];
+                    const uint2 a0 = *(const uint2*)vp, a1 = *(const uint2*)(vp + 8);
+                    vf[d] = __builtin_bit_cast(h8, make_uint4(a0.x, a0.y, a1.x, a1.y));
                 }
+#pragma unroll
+                for (int d = 0; d < DT; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[d], ph, o[d], 0, 0, 0);
+#pragma unroll
+                for (int d = 0; d < DT; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[d], pl, o[d], 0, 0, 0);
             }
-        }
     }
-    // out[row, h HD + 16 dt + 4 lg + i] for query row r0[j] + l16
-    const float sk = sink ? sink[h] * LOG2E : -INFINITY;  // in the scores' log2 units
+    // out[row, h HD + 32 d + 8 j + 4 hf + i]
+    l += __shfl_xor(l, 32, 64);
+    if (row >= T) return;
+    const float sk = sink ? sink[h] * LOG2E : -INFINITY;  // in the scores' log2 units, as m
+    const float M = fmaxf(m, sk);
+    const float sc = m == -INFINITY ? 0.0f : exp2_hw(m - M);
+    const float den = l * sc + (sk == -INFINITY ? 0.0f : exp2_hw(sk - M));
+    const float inv = den > 0.0f ? sc / den * (1.0f / PF_SCALE) : 0.0f;  // O carries the weights' scale
+    float* orow = out + (uint64_t)row * nh * HD + h * HD;
+    const float* gate = qg ? qg + (uint64_t)row * nh * 2 * HD + h * 2 * HD + HD : nullptr;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int row = r0[j] + l16;
-        if (row >= T || (j == 1 && !two)) continue;
-        const float M = fmaxf(m[j], sk);
-        const float sc = m[j] == -INFINITY ? 0.0f : exp2_hw(m[j] - M);
-        const float den = l[j] * sc + (sk == -INFINITY ? 0.0f : exp2_hw(sk - M));
-        const float inv = den > 0.0f ? sc / den * (1.0f / 16384.0f) : 0.0f;  // O carries the weights' 2^14
-        float* orow = out + (uint64_t)row * nh * HD + h * HD;
-        const float* gate = qg ? qg + (uint64_t)row * nh * 2 * HD + h * 2 * HD + HD : nullptr;
+    for (int d = 0; d < DT; d++)
 #pragma unroll
-        for (int d = 0; d < DT; d++) {
-            const int col = 16 * d + 4 * lg;
-            float4 r = make_float4(o[j][d][0] * inv, o[j][d][1] * inv, o[j][d][2] * inv, o[j][d][3] * inv);
+        for (int j = 0; j < 4; j++) {
+            const int col = 32 * d + 8 * j + 4 * hf;
+            float4 r = make_float4(o[d][4 * j] * inv, o[d][4 * j + 1] * inv, o[d][4 * j + 2] * inv, o[d][4 * j + 3] * inv);
             if (gate) {
                 r.x *= sigmoid_f(gate[col]); r.y *= sigmoid_f(gate[col + 1]);
                 r.z *= sigmoid_f(gate[col + 2]); r.w *= sigmoid_f(gate[col + 3]);
             }
             *(float4*)(orow + col) = r;
         }
-    }
 }
 
 hipError_t launch_attn_prefill(const float* q, const uint16_t* kc, const uint16_t* vc, const float* qg, float* out,
@@ -806,13 +825,14 @@ hipError_t launch_attn_prefill(const float* q, const uint16_t* kc, const uint16_
                                hipStream_t s) {
     if (t <= 0) return hipSuccess;
     const int G = nh / nkv;
-    const dim3 grid((unsigned)(((t + 15) / 16 + 1) / 2), (unsigned)nkv);  // a pair of 16-row query tiles a block
-#define PF(HD_, G_)                                                                                               \
-    if (hd == HD_ && G == G_)                                                                                     \
-        attn_prefill_kernel<HD_, G_><<<grid, dim3(64 * G_), 0, s>>>(q, kc, vc, qg, out, step, t, nh, nkv, scale,  \
-                                                                     sink, win);                                  \
-    else
-    PF(128, 1) PF(128, 2) PF(128, 4) PF(128, 8) PF(64, 1) PF(64, 2) PF(64, 4) PF(64, 8)
+#define PF(HD_, G_, HW_)                                                                                                    \
+    if (hd == HD_ && G == G_) {                                                                                             \
+        constexpr int rows = PF_Q * PF_W / HW_;                                                                             \
+        const unsigned blocks = (unsigned)(nh / HW_) * (unsigned)((t + rows - 1) / rows);                                   \
+        attn_prefill_kernel<HD_, HW_><<<dim3(blocks), dim3(64 * PF_W), 0, s>>>(q, kc, vc, qg, out, step, t, nh, nkv, scale, \
+                                                                               sink, win);                                  \
+    } else
+    PF(128, 1, 1) PF(128, 2, 2) PF(128, 4, 4) PF(128, 8, 4) PF(64, 1, 1) PF(64, 2, 2) PF(64, 4, 4) PF(64, 8, 4)
     return hipErrorInvalidValue;
 #undef PF
     return hipGetLastError();

@@ -117,3 +117,36 @@ def test_gemvn_few_positions_is_gemv(hip, ty, rows, cols):
                         assert all(np.array_equal(got[m], one[m]) for m in range(nt)), (numerics, nt)
     finally:
         hip.set_numerics(S.NUM_Q8K)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 8, 128), (8, 4, 64), (8, 2, 128), (8, 1, 64)])
+@pytest.mark.parametrize("t,pos,win", [(1, 0, 0), (31, 63, 0), (33, 100, 0), (130, 1, 48), (257, 64, 64)])
+def test_attn_prefill_rows_and_chunks(hip, nh, nkv, hd, t, pos, win):
+    """Rows at the edges of the 32-row tiles, the 64-key tiles and the window, per GQA group (heads and row tiles share a
+    block differently), against the f64 attention (float32 sums: 2e-5 of the row's norm); the same rows computed as
+    chunks of other sizes give the same bits. One query row is large, so that the running maximum jumps between tiles."""
+    n = pos + t
+    q, k, v = normal((t, nh * hd), seed=1), normal((n, nkv * hd), seed=2).astype(np.float16), normal((n, nkv * hd), seed=3).astype(np.float16)
+    q[t // 2] *= 30.0
+    kb, vb, out = up(hip, k), up(hip, v), hip.alloc(t * nh * hd * 4)
+
+    def run(chunks):
+        got, i = [], 0
+        for c in chunks:
+            step, qb = up(hip, np.array([pos + i, 0], np.int32)), up(hip, q[i:i + c])
+            hip.attn_prefill(qb, kb, vb, 0, out, step, c, nh, nkv, hd, 1.0 / np.sqrt(hd), win=win)
+            got.append(hip.get(out, np.float32, c * nh * hd).reshape(c, nh, hd))
+            i += c
+        return np.concatenate(got)
+
+    one = run([t])
+    for i in sorted({0, t // 2, t - 1}):
+        lo = max(pos + i + 1 - win, 0) if win else 0
+        for h in range(nh):
+            g = h // (nh // nkv)
+            kk, vv = (a[lo:pos + i + 1, g * hd:(g + 1) * hd].astype(np.float64) for a in (k, v))
+            s = kk @ q[i, h * hd:(h + 1) * hd].astype(np.float64) / np.sqrt(hd)
+            w = np.exp(s - s.max())
+            assert rel_l2(one[i, h], w @ vv / w.sum()) <= 2e-5, (i, h)
+    if t > 1:
+        assert np.array_equal(one.view(np.uint32), run([t // 3 + 1, t - t // 3 - 1]).view(np.uint32))
