@@ -66,23 +66,6 @@ __device__ __forceinline__ void att_range(const int* step, int t, int win, int& 
     n_pos = end + 1 - base;
 }
 
-// Eight softmax weights p (in [0, 1]) times 2^14 as f16 hi and lo parts for the P V MFMA: hi rounded toward zero two
-// at a time (v_cvt_pkrtz_f16_f32), lo the remainder (also toward zero), so hi + lo carries each weight to ~2^-21 of
-// its value and the lo parts stay normal f16 numbers down to p ~ 2^-17.
-__device__ __forceinline__ void split_p8(const float (&p)[8], h8& hi, h8& lo) {
-    uint32_t hw[4], lw[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const float a = p[2 * e] * 16384.0f, b = p[2 * e + 1] * 16384.0f;
-        const auto hh = __builtin_amdgcn_cvt_pkrtz(a, b);
-        const auto ll = __builtin_amdgcn_cvt_pkrtz(a - (float)hh[0], b - (float)hh[1]);
-        hw[e] = __builtin_bit_cast(uint32_t, hh);
-        lw[e] = __builtin_bit_cast(uint32_t, ll);
-    }
-    hi = __builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3]));
-    lo = __builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3]));
-}
-
 // ---------------- decode ----------------
 // Positions a split of a token with n_pos positions: at least one chunk of 64, so short contexts use few waves.
 __device__ __forceinline__ int split_len(int n_pos, int ns) { return max((n_pos + ns - 1) / ns, 64); }

@@ -478,9 +478,19 @@ static hipError_t gemm_t(const GemmLaunch& g, hipStream_t s) {
     a.max_tiles = g.n_tiles;
     a.dense_p = GM;
     if (!g.tiles) {
-        // a dense matrix with few row blocks (the k and v projections) takes fewer positions per tile, down to 64,
-        // until every CU has an item: the weights are then decoded more often, but no CU idles for the whole GEMM
-        while (a.dense_p > 64 && (long long)((g.dense_n + a.dense_p - 1) / a.dense_p) * nrb < ncu) a.dense_p /= 2;
+        // Positions per tile: the rounds of items over the CUs times an item's cost in 16-position MFMA tiles (its
+        // positions and about 15 for a step's decode, loads and barrier: one item a CU takes 50 / 39 / 33 us with 256 /
+        // 128 / 64 positions, Q6_K, and 52 / 36 / 28, Q4_K, at 2048 columns) is least. Q6_K, us with 256 / 128 / 64:
+        // 2048 x 4096 (o), 1501 positions 91 / 72 / 114, 512: 90 / 70 / 60, 4096: 95 / 137 / 226; 5120 x 2048 (q/k/v), 512:
+        // 50 / 39 / 62, 1501: 52 / 74 / 119, 2048: 95 / 108 / 148.
+        long long best = -1;
+        for (int p = GM; p >= 64; p /= 2) {
+            const long long items = (long long)((g.dense_n + p - 1) / p) * nrb, cost = (items + ncu - 1) / ncu * (15 + p / 16);
+            if (best < 0 || cost < best) {
+                best = cost;
+                a.dense_p = p;
+            }
+        }
         a.max_tiles = (g.dense_n + a.dense_p - 1) / a.dense_p;
     }
     // tile lists split by cost over the XCDs; an item's decode costs about as much as 4 MFMA position tiles (3, 4 and
