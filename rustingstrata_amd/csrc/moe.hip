@@ -200,6 +200,95 @@ __device__ __forceinline__ void sort_ids(const int* ids, int s0, int s1, int lan
     }
 }
 
+// From the expert totals in offs[0 .. E) (and each thread's count of bad ids): off, the tile lists and their count.
+// 1024 threads, offs complete (a barrier passed).
+__device__ __forceinline__ void sort_tiles(const SortLaunch& a, int* offs, int* tbase, int* part, int bad) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, E = a.n_expert;
+    if (wave == 0) {  // exclusive scan of the expert totals, in expert order
+        int run = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + lane;
+            const int c = e < E ? offs[e] : 0;
+            const int ic = wave_incl_scan(c);
+            if (e < E) offs[e] = run + ic - c;
+            run += __builtin_amdgcn_readlane(ic, 63);
+        }
+        if (lane == 0) offs[E] = run;
+    }
+    __syncthreads();
+    if (tid < E) tbase[tid] = (offs[tid + 1] - offs[tid] + a.chunk - 1) / a.chunk;
+    __syncthreads();
+    if (wave == 0) {  // exclusive scan of the tile counts over experts, in order
+        int trun = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + lane;
+            const int tc = e < E ? tbase[e] : 0;
+            const int itc = wave_incl_scan(tc);
+            if (e < E) tbase[e] = trun + itc - tc;
+            trun += __builtin_amdgcn_readlane(itc, 63);
+        }
+        if (lane == 0) tbase[E] = trun;
+    }
+    __syncthreads();
+    if (tid <= E) a.off[tid] = offs[tid];
+    // Tiles: expert e's slots off[e] .. off[e + 1] in chunks of a.chunk positions.
+    if (tid < E) {
+        const int c = offs[tid + 1] - offs[tid], tb = tbase[tid];
+        for (int j = 0; j * a.chunk < c; j++) {
+            const uint64_t m0 = (uint64_t)(offs[tid] + j * a.chunk), cn = (uint64_t)min(a.chunk, c - j * a.chunk);
+            for (int m = 0; m < a.n_mats; m++) {
+                uint64_t* tl = a.tiles + 2 * ((uint64_t)m * a.max_tiles + tb + j);
+                tl[0] = a.bases[m] + (uint64_t)tid * a.strides[m];
+                tl[1] = m0 | cn << 32;
+            }
+        }
+    }
+    if (a.err) {
+        bad = __builtin_amdgcn_readlane(wave_incl_scan(bad), 63);
+        if (lane == 0) part[wave] = bad;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        *a.n_tiles = tbase[E];
+        if (a.err) {
+            int b = 0;
+            for (int w = 0; w < 16; w++) b += part[w];
+            *a.err = b;
+        }
+    }
+}
+
+// This wave's pairs s0 .. s1 (ids in eu) in order: h[e] is expert e's next slot.
+__device__ __forceinline__ void sort_walk(const SortLaunch& a, const int (&eu)[SORT_U], int s0, int s1, int lane, int* h) {
+    const int E = a.n_expert;
+#pragma unroll
+    for (int u = 0; u < SORT_U; u++) {
+        const int c0 = s0 + 64 * u;
+        if (c0 >= s1) break;
+        const int i = c0 + lane;
+        const bool live = i < s1;
+        const int e = eu[u];
+        const bool ok = live && e >= 0 && e < E;
+        const int key = ok ? e : (live ? 2046 : 2047);
+        uint64_t peers = ~0ull;
+#pragma unroll
+        for (int b = 0; b < 11; b++) {
+            const uint64_t m = __ballot((key >> b) & 1);
+            peers &= ((key >> b) & 1) ? m : ~m;
+        }
+        const int rank = __popcll(peers & ((1ull << lane) - 1));
+        const int slot = ok ? h[e] + rank : -1;
+        __builtin_amdgcn_wave_barrier();
+        if (ok && rank == 0) h[e] += __popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (live) {
+            a.inv[i] = slot;
+            if (ok) a.xrow[slot] = i / a.k;
+        }
+    }
+}
+
 __global__ __launch_bounds__(1024) void sort_count_kernel(SortLaunch a, int W) {
     __shared__ int hist[SORT_WAVES][SORT_MAX_E];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, E = a.n_expert;
@@ -270,58 +359,7 @@ __global__ __launch_bounds__(1024) void sort_scan_kernel(SortLaunch a, int W) {
     if (a.err)
         for (int w = tid; w < W; w += 1024) bad += cnt[L + w];
     __syncthreads();
-    if (wave == 0) {  // exclusive scan of the expert totals, in expert order
-        int run = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + lane;
-            const int c = e < E ? offs[e] : 0;
-            const int ic = wave_incl_scan(c);
-            if (e < E) offs[e] = run + ic - c;
-            run += __builtin_amdgcn_readlane(ic, 63);
-        }
-        if (lane == 0) offs[E] = run;
-    }
-    __syncthreads();
-    if (tid < E) tbase[tid] = (offs[tid + 1] - offs[tid] + a.chunk - 1) / a.chunk;
-    __syncthreads();
-    if (wave == 0) {  // exclusive scan of the tile counts over experts, in order
-        int trun = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + lane;
-            const int tc = e < E ? tbase[e] : 0;
-            const int itc = wave_incl_scan(tc);
-            if (e < E) tbase[e] = trun + itc - tc;
-            trun += __builtin_amdgcn_readlane(itc, 63);
-        }
-        if (lane == 0) tbase[E] = trun;
-    }
-    __syncthreads();
-    if (tid <= E) a.off[tid] = offs[tid];
-    // Tiles: expert e's slots off[e] .. off[e + 1] in chunks of a.chunk positions.
-    if (tid < E) {
-        const int c = offs[tid + 1] - offs[tid], tb = tbase[tid];
-        for (int j = 0; j * a.chunk < c; j++) {
-            const uint64_t m0 = (uint64_t)(offs[tid] + j * a.chunk), cn = (uint64_t)min(a.chunk, c - j * a.chunk);
-            for (int m = 0; m < a.n_mats; m++) {
-                uint64_t* tl = a.tiles + 2 * ((uint64_t)m * a.max_tiles + tb + j);
-                tl[0] = a.bases[m] + (uint64_t)tid * a.strides[m];
-                tl[1] = m0 | cn << 32;
-            }
-        }
-    }
-    if (a.err) {
-        bad = __builtin_amdgcn_readlane(wave_incl_scan(bad), 63);
-        if (lane == 0) part[wave] = bad;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        *a.n_tiles = tbase[E];
-        if (a.err) {
-            int b = 0;
-            for (int w = 0; w < 16; w++) b += part[w];
-            *a.err = b;
-        }
-    }
+    sort_tiles(a, offs, tbase, part, bad);
 }
 
 __global__ __launch_bounds__(1024) void sort_scatter_kernel(SortLaunch a, int W) {
@@ -335,36 +373,57 @@ __global__ __launch_bounds__(1024) void sort_scatter_kernel(SortLaunch a, int W)
     for (int e = lane; e < E; e += 64) hist[wave][e] = a.off[e] + a.scratch[(uint64_t)e * W + gw];
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    sort_walk(a, eu, s0, s1, lane, hist[wave]);
+}
+
+// Up to 16 waves of pairs (4096: a 512-token prompt at top 8): the three kernels' work in one block, the wave counts and
+// their prefixes in LDS. A launch that small is all latency: 14.3 us of traced kernel time for the
+// three, 5.5 here (216 pairs; the 27-token MoE block 127 -> 120 us).
+__global__ __launch_bounds__(1024) void sort_one_kernel(SortLaunch a, int W) {
+    __shared__ int hist[SORT_WAVES][SORT_MAX_E];
+    __shared__ int part[16];
+    __shared__ int offs[SORT_MAX_E + 1], tbase[SORT_MAX_E + 1];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, E = a.n_expert, N = a.t * a.k;
+    const int s0 = min(N, wave * SORT_SEG), s1 = min(N, s0 + SORT_SEG);
+    int eu[SORT_U];
+    sort_ids(a.ids, s0, s1, lane, eu);
+    for (int i = tid; i < W * E; i += 1024) hist[i / E][i % E] = 0;
+    __syncthreads();
+    int bad = 0;
 #pragma unroll
     for (int u = 0; u < SORT_U; u++) {
-        const int c0 = s0 + 64 * u;
-        if (c0 >= s1) break;
-        const int i = c0 + lane;
-        const bool live = i < s1;
-        const int e = eu[u];
-        const bool ok = live && e >= 0 && e < E;
-        const int key = ok ? e : (live ? 2046 : 2047);
-        uint64_t peers = ~0ull;
-#pragma unroll
-        for (int b = 0; b < 11; b++) {
-            const uint64_t m = __ballot((key >> b) & 1);
-            peers &= ((key >> b) & 1) ? m : ~m;
-        }
-        const int rank = __popcll(peers & ((1ull << lane) - 1));
-        const int slot = ok ? hist[wave][e] + rank : -1;
-        __builtin_amdgcn_wave_barrier();
-        if (ok && rank == 0) hist[wave][e] += __popcll(peers);
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        if (live) {
-            a.inv[i] = slot;
-            if (ok) a.xrow[slot] = i / a.k;
+        if (s0 + 64 * u + lane < s1) {
+            const int e = eu[u];
+            if (e >= 0 && e < E) atomicAdd(&hist[wave][e], 1);
+            else bad++;
         }
     }
+    __syncthreads();
+    if (tid < E) {  // the waves' counts into exclusive prefixes within the expert
+        int run = 0;
+        for (int w = 0; w < W; w++) {
+            const int c = hist[w][tid];
+            hist[w][tid] = run;
+            run += c;
+        }
+        offs[tid] = run;
+    }
+    __syncthreads();
+    sort_tiles(a, offs, tbase, part, bad);
+    __syncthreads();
+    if (wave < W)
+        for (int e = lane; e < E; e += 64) hist[wave][e] += offs[e];
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (wave < W) sort_walk(a, eu, s0, s1, lane, hist[wave]);
 }
 
 hipError_t launch_sort(const SortLaunch& a, hipStream_t s) {
     const int W = sort_waves(a.t * a.k), blocks = (W + SORT_WAVES - 1) / SORT_WAVES;
+    if (blocks <= 1) {
+        sort_one_kernel<<<1, 1024, 0, s>>>(a, W);
+        return hipGetLastError();
+    }
     sort_count_kernel<<<blocks, 1024, 0, s>>>(a, W);
     sort_scan_kernel<<<1, 1024, 0, s>>>(a, W);
     sort_scatter_kernel<<<blocks, 1024, 0, s>>>(a, W);

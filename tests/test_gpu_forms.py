@@ -150,3 +150,32 @@ def test_attn_prefill_rows_and_chunks(hip, nh, nkv, hd, t, pos, win):
             assert rel_l2(one[i, h], w @ vv / w.sum()) <= 2e-5, (i, h)
     if t > 1:
         assert np.array_equal(one.view(np.uint32), run([t // 3 + 1, t - t // 3 - 1]).view(np.uint32))
+
+
+# one block up to 4096 pairs, three launches beyond
+@pytest.mark.parametrize("t,k,E,chunk", [(1, 1, 1, 64), (3, 2, 512, 64), (512, 8, 128, 64), (512, 8, 512, 256), (513, 8, 128, 64)])
+def test_moe_sort_forms(hip, t, k, E, chunk):
+    """The device sort on both sides of its one-block form against numpy's stable sort: off, xrow, inv, the tiles and the
+    count of ids out of range (which get no slot)."""
+    rng = np.random.default_rng(t + E)
+    ids = rng.integers(0, E, (t, k)).astype(np.int32)
+    ids.reshape(-1)[:: 37] = E // 2
+    bad = rng.random(t * k) < 0.02
+    flat = ids.reshape(-1)
+    flat[bad] = np.where(rng.random(int(bad.sum())) < 0.5, -1, E)
+    mt = t * k // chunk + E
+    off, xrow, inv, ntd, err, tiles = (hip.alloc(b) for b in (4 * (E + 1), 4 * t * k, 4 * t * k, 4, 4, 16 * mt))
+    hip.moe_sort(up(hip, flat), t, k, E, off, xrow, inv, [(1 << 20, 4096)], tiles, mt, ntd, err_dev=err, chunk=chunk)
+    good = np.flatnonzero(~bad)
+    order = good[np.argsort(flat[good], kind="stable")]
+    want_inv = np.full(t * k, -1, np.int32)
+    want_inv[order] = np.arange(len(order))
+    cnt = np.bincount(flat[good], minlength=E)
+    want_off = np.concatenate([[0], np.cumsum(cnt)])
+    assert np.array_equal(hip.get(off, np.int32, E + 1), want_off)
+    assert np.array_equal(hip.get(inv, np.int32, t * k), want_inv)
+    assert np.array_equal(hip.get(xrow, np.int32, t * k)[:len(order)], order // k)
+    assert hip.get(err, np.int32, 1)[0] == bad.sum()
+    want = [((1 << 20) + 4096 * e, (want_off[e] + j) | min(chunk, int(cnt[e]) - j) << 32) for e in range(E) for j in range(0, int(cnt[e]), chunk)]
+    assert hip.get(ntd, np.int32, 1)[0] == len(want)
+    assert [tuple(r) for r in hip.get(tiles, np.uint64, 2 * len(want)).reshape(-1, 2).tolist()] == [(int(a), int(b)) for a, b in want]
