@@ -140,23 +140,24 @@ __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_kernel(NormRope a) {
 // per head (the heads' sequential chains run side by side); each wave then takes 16 consecutive heads, a lane per
 // rope pair (i, i + 64), recomputing the pair's angle only when the position changes. The arithmetic is
 // norm_rope_kernel's, so both kernels give the same bits.
+// (The value rows are read where they are stored, not staged: 33 KB of LDS a block, four a CU instead of two; 1501 tokens x
+// 36 heads 31.3 -> 28.6 us.)
 constexpr int NR_MANY = 64, NR_P = 129;  // heads a block; LDS pitch of a staged head (bank spread for the sums)
 __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_many_kernel(NormRope a) {
-    __shared__ float xs[NR_MANY][NR_P], vs[NR_MANY][NR_P];
+    __shared__ float xs[NR_MANY][NR_P];
     __shared__ float ssq[NR_MANY];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int total = a.qrows + a.rows, g0 = (int)blockIdx.x * NR_MANY;
     const float qw0 = a.qrows ? a.qw[lane] : 0.0f, qw1 = a.qrows ? a.qw[lane + 64] : 0.0f;
     const float kw0 = a.rows ? a.w[lane] : 0.0f, kw1 = a.rows ? a.w[lane + 64] : 0.0f;
     // 16-byte chunk c = tid + 256 u of the block: head c / 32, values 4 (c % 32) ..
-    float4 xv[8], vv[8];
+    float4 xv[8];
 #pragma unroll
     for (int u = 0; u < 8; u++) {
         const int c = tid + 256 * u, j = c >> 5, g = g0 + j;
         if (g < total) {
             const NrHead h = nr_head(a, g);
             xv[u] = *(const float4*)(h.xr + 4 * (c & 31));
-            if (h.vr) vv[u] = *(const float4*)(h.vr + 4 * (c & 31));
         }
     }
 #pragma unroll
@@ -164,9 +165,6 @@ __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_many_kernel(NormRope 
         const int c = tid + 256 * u, j = c >> 5, g = g0 + j, i = 4 * (c & 31);
         if (g < total) {
             xs[j][i] = xv[u].x; xs[j][i + 1] = xv[u].y; xs[j][i + 2] = xv[u].z; xs[j][i + 3] = xv[u].w;
-            if (g >= a.qrows && a.kc) {
-                vs[j][i] = vv[u].x; vs[j][i + 1] = vv[u].y; vs[j][i + 2] = vv[u].z; vs[j][i + 3] = vv[u].w;
-            }
         }
     }
     __syncthreads();
@@ -207,8 +205,8 @@ __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_many_kernel(NormRope 
             const uint64_t e = ((uint64_t)pos * h.per + h.b % h.per) * 128;
             a.kc[e + lane] = f32_to_f16_bits(o0);
             a.kc[e + lane + 64] = f32_to_f16_bits(o1);
-            a.vc[e + lane] = f32_to_f16_bits(vs[j][lane]);
-            a.vc[e + lane + 64] = f32_to_f16_bits(vs[j][lane + 64]);
+            a.vc[e + lane] = f32_to_f16_bits(h.vr[lane]);
+            a.vc[e + lane + 64] = f32_to_f16_bits(h.vr[lane + 64]);
         }
     }
 }
