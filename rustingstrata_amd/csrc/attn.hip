@@ -807,6 +807,7 @@ hipError_t launch_attn_prefill(const float* q, const uint16_t* kc, const uint16_
                                const int* step, int t, int nh, int nkv, int hd, float scale, const float* sink, int win,
                                hipStream_t s) {
     if (t <= 0) return hipSuccess;
+    if (nkv > 65535) return hipErrorInvalidValue;  // (a cache row's bytes fit the 24-bit multiplies)
     const int G = nh / nkv;
 #define PF(HD_, G_, HW_)                                                                                                    \
     if (hd == HD_ && G == G_) {                                                                                             \

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_kernel(NormRope a) {
 }
 
 // Many heads of 128 values, all rotated (a prefill chunk): a block takes NR_MANY heads. Its threads stage the heads
-// (and the value rows of stored key heads) in LDS with every load issued at once; wave 0 then sums the squares a lane
+// in LDS with every load issued at once; wave 0 then sums the squares a lane
 // per head (the heads' sequential chains run side by side); each wave then takes 16 consecutive heads, a lane per
 // rope pair (i, i + 64), recomputing the pair's angle only when the position changes. The arithmetic is
 // norm_rope_kernel's, so both kernels give the same bits.

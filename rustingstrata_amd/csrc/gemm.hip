@@ -530,8 +530,8 @@ __global__ __launch_bounds__(256, 3) void gemm_q8_0_kernel(GemmArgs a) {
     // row blocks' weights stay in its L2 while X streams by
     const int nrb = (a.rows + Q8_ROWS - 1) / Q8_ROWS;
     const long long total = (long long)nrb * ntiles, per = (total + NXCD - 1) / NXCD;
-    const long long id = (long long)(blockIdx.x % NXCD) * per + blockIdx.x / NXCD;
-    if ((long long)(blockIdx.x / NXCD) >= per || id >= total) return;
+    const long long at = blockIdx.x / NXCD + (long long)blockIdx.y * (gridDim.x / NXCD), id = (blockIdx.x % NXCD) * per + at;
+    if (at >= per || id >= total) return;
     const int rb = (int)(id / ntiles), tile = (int)(id - (long long)rb * ntiles), n0 = rb * Q8_ROWS;
     uint64_t w;
     int m0, cnt;
@@ -655,9 +655,9 @@ static hipError_t gemm_q8_0(const GemmLaunch& g, hipStream_t s) {
     a.rb = row_bytes(Q8_0, g.cols);
     a.max_tiles = g.tiles ? g.n_tiles : (g.dense_n + Q8_POS - 1) / Q8_POS;
     const long long total = (long long)((g.rows + Q8_ROWS - 1) / Q8_ROWS) * a.max_tiles;
-    const long long grid = (total + NXCD - 1) / NXCD * NXCD;
-    if (grid >= (1ll << 31)) return hipErrorInvalidValue;
-    gemm_q8_0_kernel<<<dim3((unsigned)grid), 256, 0, s>>>(a);
+    const long long grid = std::min((total + NXCD - 1) / NXCD * NXCD, 1ll << 30), ny = (total + grid - 1) / std::max(grid, 1ll);
+    if (ny > 65535) return hipErrorInvalidValue;
+    gemm_q8_0_kernel<<<dim3((unsigned)grid, (unsigned)ny), 256, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -371,7 +371,7 @@ hipError_t launch_gemv_few(const GemvLaunch& g, hipStream_t s) {
 bool gemm_few_takes(const GemmLaunch& g) {
     if (g.ty == Q8_0) return false;
     if (!g.tiles) return g.dense_n <= FPM || few_dense_items(g.rows, g.dense_n) <= FEW_DENSE_ITEMS;
-    if (!g.small) return false;
+    if (!g.small || (long long)((g.rows + 15) / 16) * g.n_tiles >= (1ll << 31)) return false;
     const bool sa = g.ty == Q4_K || g.ty == Q5_K || g.ty == IQ4_XS || g.ty == IQ3_S;
     if (g.xrow) return g.n_x <= (sa ? 32 : 128);
     return g.n_x <= (!sa ? 1024 : g.ty == IQ4_XS || g.ty == IQ3_S ? 320 : 128) && g.n_x <= 12ll * g.n_tiles;
