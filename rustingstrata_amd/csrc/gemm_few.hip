@@ -39,12 +39,29 @@ constexpr int FPP = FPM + 4;  // floats of a term row (16-byte pad: rows start i
 constexpr long long FEW_DENSE_BLOCK_ITEMS = 1280, FEW_DENSE_ITEMS = 2048;
 long long few_dense_items(int rows, int n) { return (long long)((rows + 15) / 16) * ((n + FPM - 1) / FPM); }
 // Tile lists with SMALL_TILES, 128 experts, top 8, 2048 x 768: gate/up by the tokens gathered from (27 / 100 / 200
-// tokens): Q2_K 66 -> 40 / 94 -> 67 / 95 -> 92, Q3_K 112 -> 65 / 157 -> 110 / 157 -> 137, IQ2_XXS 100 -> 57 / 140 -> 94 /
-// 141 -> 118; the scale-after types, whose close is heavier per tile, only up to 32 tokens: Q5_K 64 -> 53 / 94 -> 103,
-// Q4_K 59 -> 51 / 86 -> 94, IQ4_XS 72 -> 54 / 102 -> 98 (64 tokens: 82 -> 87). Down by the rows of X (216 / 800 / 1600):
-// Q3_K 52 -> 35 / 76 -> 61 / 76 -> 63, Q6_K 50 -> 35 / 72 -> 61 / 72 -> 62; IQ4_XS 40 -> 37 (320: 47 -> 42, 512: 50 ->
-// 54), IQ3_S 47 -> 39; Q4_K 128: 25 -> 23, 216: 33 -> 37, Q5_K 27 -> 24, 36 -> 38. At most 12 rows a tile slot: with
-// fewer, fuller tiles every 16 positions would decode the weights again.
+// tokens): Q3_K 81 -> 65 / 120 -> 110 / 122 -> 138 (128 tokens: 121 -> 121), IQ2_XXS 69 -> 57 / 103 -> 95 / 105 -> 119
+// (128: 104 -> 103), Q2_K 48 -> 42 / 67 -> 67 / 69 -> 92 (48: 57 -> 55, 64: 58 -> 62); the scale-after types, whose close
+// is heavier per tile, only up to 32 tokens: Q5_K 64 -> 53 / 94 -> 103, Q4_K 59 -> 51 / 86 -> 94, IQ4_XS 72 -> 54 / 102
+// -> 98 (64 tokens: 82 -> 87). Down by the rows of X (216 / 512 / 800): Q3_K 43 -> 37 / 52 -> 51 / 57 -> 61, IQ2_XXS 46 ->
+// 38 / 58 -> 54 / 63 -> 64, Q2_K 27 -> 24 / 32 -> 35 / 35 -> 44 (384: 31 -> 31), Q6_K 50 -> 35 / - / 72 -> 61 (1600: 72
+// -> 62); IQ4_XS 40 -> 37 (320: 47 -> 42, 512: 50 -> 54), IQ3_S 47 -> 39; Q4_K 128: 25 -> 23, 216: 33 -> 37, Q5_K 27 ->
+// 24, 36 -> 38. At most 12 rows a tile slot: with fewer, fuller tiles every 16 positions would decode the weights again.
+int few_gathered(int ty) {
+    switch (ty) {
+    case Q3_K: case Q6_K: case IQ2_XXS: return 128;
+    case Q2_K: return 48;
+    default: return 32;
+    }
+}
+int few_rows(int ty) {
+    switch (ty) {
+    case Q6_K: return 1024;
+    case Q3_K: case IQ2_XXS: return 512;
+    case Q2_K: return 384;
+    case IQ3_S: case IQ4_XS: return 320;
+    default: return 128;
+    }
+}
 }  // namespace
 
 template <int T> struct FewFmt : GemmPlanes<T> {
@@ -372,9 +389,8 @@ bool gemm_few_takes(const GemmLaunch& g) {
     if (g.ty == Q8_0) return false;
     if (!g.tiles) return g.dense_n <= FPM || few_dense_items(g.rows, g.dense_n) <= FEW_DENSE_ITEMS;
     if (!g.small || (long long)((g.rows + 15) / 16) * g.n_tiles >= (1ll << 31)) return false;
-    const bool sa = g.ty == Q4_K || g.ty == Q5_K || g.ty == IQ4_XS || g.ty == IQ3_S;
-    if (g.xrow) return g.n_x <= (sa ? 32 : 128);
-    return g.n_x <= (!sa ? 1024 : g.ty == IQ4_XS || g.ty == IQ3_S ? 320 : 128) && g.n_x <= 12ll * g.n_tiles;
+    if (g.xrow) return g.n_x <= few_gathered(g.ty);
+    return g.n_x <= few_rows(g.ty) && g.n_x <= 12ll * g.n_tiles;
 }
 
 hipError_t launch_gemm_few(const GemmLaunch& g, hipStream_t s) {

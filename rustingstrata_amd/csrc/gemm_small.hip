@@ -3,13 +3,16 @@
 // kernels gemmi_q / gemms_*, src/cuda/kernels.cu:1355-1497, chosen by tile size in src/cuda/mod.rs:587-620).
 //
 // With few positions a block's super-block step is short (the 16 rows a wave decodes, then one or two MFMA tile
-// pairs), so a weight load issued one step ahead does not land in time. This kernel keeps two steps in flight:
+// pairs), so a weight load issued one step ahead does not land in time. The types whose kernel fits 128 registers
+// (small_two) run two blocks a CU, each one step ahead, and wait for all loads at a step's end; the others run one
+// block a CU that keeps two steps in flight:
 //   * a block takes 64 positions x 128 weight rows (8 waves, 16 rows each, as gemm_kernel; pair mode 64 gate + 64 up);
 //   * X rows and their scales sit in a ring of three LDS buffers, raw weights in two per wave, and step g issues the
-//     loads of step g + 2 (X and scales between its decode units, its own weight rows right after its decode);
+//     loads of step g + 2 (X and scales between its decode units, its own weight rows right after its decode); with
+//     two blocks a CU, two X buffers, one of raw rows, and the loads of step g + 1;
 //   * every wave issues the same number of loads each step (positions past a tile's count load its first row, weight
 //     chunks a row does not need reload its first chunk into the wave's padded region), so the end of step g waits
-//     with vmcnt for step g + 1's loads alone, and the block barrier does not drain step g + 2's;
+//     with vmcnt for step g + 1's loads alone, and the block barrier does not drain step g + 2's (one block a CU);
 //   * a tile of more than 64 positions runs as consecutive 64-position chunks (any tile list is computed whole; the
 //     fast case is a tile list built with chunks of 64, strata_moe_sort's chunk = 64).
 // Each wave keeps its own copy of a step's 64 X scales (one 4-byte load-to-LDS per lane), so scales need no barrier.
@@ -28,11 +31,19 @@ constexpr int SW = 8;                   // waves per block
 constexpr int STT = SM / 16;            // MFMA position tiles per block
 constexpr int SXB = SM * 256;           // bytes of one X buffer
 constexpr int SXI = SM * 16 / 64 / SW;  // X load instructions per wave and step
-constexpr int NXB = 3;                  // X (and scale) buffers: steps g, g + 1, g + 2
 constexpr int SDX = SW * SM;            // floats of one scale buffer (a copy per wave)
 }  // namespace
 
+// Two blocks a CU, each one step ahead (X in 2 slots, raw rows in 1), for the types whose kernel fits 128 registers: the
+// other block's waves cover a step's waits better than a second step in flight does. 512-token GEMMs over 128 experts,
+// us with one block / two: Q2_K gate/up 114 / 81, IQ2_XXS 168 / 121, Q3_K down 89 / 70 (1000 tokens 141 / 109, 204 / 148,
+// 115 / 91); the others spill and lose (Q6_K down 84 / 99, IQ4_XS gate/up 128 / 261).
+__host__ __device__ constexpr bool small_two(int T) { return T == Q2_K || T == Q3_K || T == IQ2_XXS; }
+
 template <int T> struct SmallFmt : GemmPlanes<T> {
+    static constexpr bool TWO = small_two(T);
+    static constexpr int NXB = TWO ? 2 : 3;                          // X (and scale) buffers: steps g, g + 1 (, g + 2)
+    static constexpr int NWB = TWO ? 1 : 2;                          // raw weight buffers
     static constexpr int WI = (16 * GemmPlanes<T>::NCH + 63) / 64;  // weight load instructions per wave and step
     static constexpr int WREG = 64 * WI * 16;                        // LDS bytes of a wave's raw rows (whole instructions)
     static constexpr int WBUF = SW * WREG;                           // bytes of one raw weight buffer
@@ -40,21 +51,22 @@ template <int T> struct SmallFmt : GemmPlanes<T> {
 };
 
 template <int T>
-__global__ __launch_bounds__(64 * SW, 1) void gemm_small_kernel(GemmArgs a) {
+__global__ __launch_bounds__(64 * SW, SmallFmt<T>::TWO ? 4 : 1) void gemm_small_kernel(GemmArgs a) {
     using F = SmallFmt<T>;
     constexpr int NP = F::NP, SBB = sb_bytes(T), NCH = F::NCH, RAWP = F::RAWP, WI = F::WI, WREG = F::WREG,
-                  WBUF = F::WBUF, NLOAD = F::NLOAD;
+                  WBUF = F::WBUF, NLOAD = F::NLOAD, NXB = F::NXB, NWB = F::NWB;
+    constexpr bool TWO = F::TWO;
     constexpr int P_HI = 0, P_LO = F::HI ? 1 : 0, P_M = F::HI ? 2 : 1;
     constexpr bool IQ = T == IQ2_XXS || T == IQ3_S;
     static_assert(NCH <= 15 && WI <= 8, "chunk numbers of a lane's weight instructions fit one word");
     static_assert(SBB < 225, "the no-chunk number 15 lands past every super-block");
     static_assert(SXI == 2, "the decode hook issues two X instructions and the scales");
     extern __shared__ __align__(16) uint8_t smem[];
-    // LDS: [X: NXB x SXB][scales: NXB x SDX floats][raw W: 2 x WBUF][IqTables]
+    // LDS: [X: NXB x SXB][scales: NXB x SDX floats][raw W: NWB x WBUF][IqTables]
     int8_t* xs = (int8_t*)smem;
     float* dxs = (float*)(smem + NXB * SXB);
     uint8_t* raw = (uint8_t*)(dxs + NXB * SDX);
-    IqTables* tab = (IqTables*)(raw + 2 * WBUF);
+    IqTables* tab = (IqTables*)(raw + NWB * WBUF);
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int cols = a.cols, nsb = cols / 256;
@@ -75,8 +87,8 @@ __global__ __launch_bounds__(64 * SW, 1) void gemm_small_kernel(GemmArgs a) {
     int mine = 0, ns = -1;
     if (a.bal >= 0 && ntiles <= 64 * SW) {
         int ia, ib;
-        static_assert(PLAN_INTS * 4 <= SXB, "the plan fits X slot 2, first written after the first barrier");
-        ns = plan_items<SW>(cnt0, ntiles, nrb, a.bal, 1, 0, ibeg, gstep, (int*)(xs + 2 * SXB), ia, ib, mine);
+        static_assert(PLAN_INTS * 4 <= SXB, "the plan fits the last X slot, first written after the first barrier");
+        ns = plan_items<SW>(cnt0, ntiles, nrb, a.bal, 1, 0, ibeg, gstep, (int*)(xs + (NXB - 1) * SXB), ia, ib, mine);
     }
     const bool mine_ok = ns >= 0;
     const int nitems = mine_ok ? ns : ibeg < total ? (total - ibeg + gstep - 1) / gstep : 0;
@@ -377,78 +389,127 @@ __global__ __launch_bounds__(64 * SW, 1) void gemm_small_kernel(GemmArgs a) {
             for (int q = 0; q < 4; q++) acc[i][q] = 0.0f;
     };
 
-    // The step stream: cur (step g), q1 (step g + 1) and the load state L (step g + 2: item index kL, super-block sL).
-    struct Step {
-        Item it;
-        uint32_t rbeg;
-        int s;
-    };
-    int kL = -1, pcL = 0, sL = 0;
-    Item iL = next_item(kL, pcL, Item{0, 0, 0, 0, 0});
-    if (iL.cnt == 0) return;  // no work: no load was issued
-    Addr aL = addr_of(iL);
-    auto advance = [&]() __attribute__((always_inline)) {
-        if (++sL == nsb) {
-            sL = 0;
-            iL = next_item(kL, pcL, iL);
-            if (iL.cnt) aL = addr_of(iL);
-        }
-    };
-    auto issue_all = [&](int xb, int wb) __attribute__((always_inline)) {
-        load_x(aL, sL, xb, 0);
-        load_x(aL, sL, xb, 1);
-        load_dx(aL, sL, xb);
-        load_w(iL, aL, sL, wb);
-    };
-    // prologue: steps 0 and 1
-    Step cur{iL, aL.rbeg, sL};
-    issue_all(0, 0);
-    advance();
-    Step q1{iL, aL.rbeg, sL};
-    if (iL.cnt) {
-        issue_all(1, 1);
-        advance();
-        wait_vm<NLOAD>();
-    } else {
-        wait_vm<0>();
-    }
-    __syncthreads();  // the IQ tables and step 0's X
-
-    int xb = 0, wb = 0;  // buffers of step g
-    while (true) {
-        const bool l2 = iL.cnt != 0;  // step g + 2 exists
-        const int xb2 = xb == 0 ? 2 : xb - 1;
-        decode(cur.rbeg, cur.s, wb, [&](int kk) __attribute__((always_inline)) {
-            if (l2) {
-                if (kk < SXI) load_x(aL, sL, xb2, kk);
-                else if (kk == SXI) load_dx(aL, sL, xb2);
+    if constexpr (TWO) {
+        // One step ahead: cur (step g) and the load state L (step g + 1: item index kL, super-block sL).
+        int kL = -1, pcL = 0, sL = 0;
+        Item iL = next_item(kL, pcL, Item{0, 0, 0, 0, 0});
+        if (iL.cnt == 0) return;  // no work: no load was issued
+        Addr aL = addr_of(iL);
+        load_x(aL, 0, 0, 0);
+        load_x(aL, 0, 0, 1);
+        load_dx(aL, 0, 0);
+        load_w(iL, aL, 0, 0);
+        Item cur = iL;
+        uint32_t rbeg = aL.rbeg;
+        int s = 0;
+        auto advance = [&]() __attribute__((always_inline)) {
+            if (++sL == nsb) {
+                sL = 0;
+                iL = next_item(kL, pcL, iL);
+                if (iL.cnt) aL = addr_of(iL);
             }
-        });
-        wait_lds();  // this wave's reads of its raw rows are done: step g + 2's rows take the buffer
-        if (l2) load_w(iL, aL, sL, wb);
-        tiles(xb, (cur.it.cnt + 15) >> 4);
-        const bool last = cur.s + 1 == nsb;
-        if (last) store(cur.it, xb);
-        if (q1.it.cnt == 0) break;  // step g was the block's last
-        cur = q1;
-        if (l2) {
-            q1 = Step{iL, aL.rbeg, sL};
+        };
+        advance();
+        wait_vm<0>();
+        __syncthreads();  // the IQ tables and step 0's X
+        int xb = 0;
+        while (true) {
+            const bool more = iL.cnt != 0;  // step g + 1 exists
+            decode(rbeg, s, 0, [&](int kk) __attribute__((always_inline)) {
+                if (more) {
+                    if (kk < SXI) load_x(aL, sL, xb ^ 1, kk);
+                    else if (kk == SXI) load_dx(aL, sL, xb ^ 1);
+                }
+            });
+            wait_lds();  // this wave's reads of its raw rows are done: step g + 1's rows take them over
+            asm volatile("" : : : "memory");
+            if (more) load_w(iL, aL, sL, 0);
+            tiles(xb, (cur.cnt + 15) >> 4);
+            if (s + 1 == nsb) store(cur, xb);
+            if (!more) break;
+            cur = iL;
+            rbeg = aL.rbeg;
+            s = sL;
             advance();
-        } else {
-            q1.it.cnt = 0;
+            wait_vm<0>();
+            lds_barrier();
+            xb ^= 1;
         }
-        // step g + 1's loads have landed (step g + 2's may still fly, unless an item's stores were issued after them)
-        if (last || !l2) wait_vm<0>();
-        else wait_vm<NLOAD>();
-        lds_barrier();
-        xb = xb == 2 ? 0 : xb + 1;
-        wb ^= 1;
+    } else {
+        // The step stream: cur (step g), q1 (step g + 1) and the load state L (step g + 2: item index kL, super-block sL).
+        struct Step {
+            Item it;
+            uint32_t rbeg;
+            int s;
+        };
+        int kL = -1, pcL = 0, sL = 0;
+        Item iL = next_item(kL, pcL, Item{0, 0, 0, 0, 0});
+        if (iL.cnt == 0) return;  // no work: no load was issued
+        Addr aL = addr_of(iL);
+        auto advance = [&]() __attribute__((always_inline)) {
+            if (++sL == nsb) {
+                sL = 0;
+                iL = next_item(kL, pcL, iL);
+                if (iL.cnt) aL = addr_of(iL);
+            }
+        };
+        auto issue_all = [&](int xb, int wb) __attribute__((always_inline)) {
+            load_x(aL, sL, xb, 0);
+            load_x(aL, sL, xb, 1);
+            load_dx(aL, sL, xb);
+            load_w(iL, aL, sL, wb);
+        };
+        // prologue: steps 0 and 1
+        Step cur{iL, aL.rbeg, sL};
+        issue_all(0, 0);
+        advance();
+        Step q1{iL, aL.rbeg, sL};
+        if (iL.cnt) {
+            issue_all(1, 1);
+            advance();
+            wait_vm<NLOAD>();
+        } else {
+            wait_vm<0>();
+        }
+        __syncthreads();  // the IQ tables and step 0's X
+
+        int xb = 0, wb = 0;  // buffers of step g
+        while (true) {
+            const bool l2 = iL.cnt != 0;  // step g + 2 exists
+            const int xb2 = xb == 0 ? 2 : xb - 1;
+            decode(cur.rbeg, cur.s, wb, [&](int kk) __attribute__((always_inline)) {
+                if (l2) {
+                    if (kk < SXI) load_x(aL, sL, xb2, kk);
+                    else if (kk == SXI) load_dx(aL, sL, xb2);
+                }
+            });
+            wait_lds();  // this wave's reads of its raw rows are done: step g + 2's rows take the buffer
+            if (l2) load_w(iL, aL, sL, wb);
+            tiles(xb, (cur.it.cnt + 15) >> 4);
+            const bool last = cur.s + 1 == nsb;
+            if (last) store(cur.it, xb);
+            if (q1.it.cnt == 0) break;  // step g was the block's last
+            cur = q1;
+            if (l2) {
+                q1 = Step{iL, aL.rbeg, sL};
+                advance();
+            } else {
+                q1.it.cnt = 0;
+            }
+            // step g + 1's loads have landed (step g + 2's may still fly, unless an item's stores were issued after them)
+            if (last || !l2) wait_vm<0>();
+            else wait_vm<NLOAD>();
+            lds_barrier();
+            xb = xb == 2 ? 0 : xb + 1;
+            wb ^= 1;
+        }
     }
 }
 
 template <int T>
 static size_t gemm_small_smem() {
-    size_t b = (size_t)NXB * SXB + (size_t)NXB * SDX * 4 + 2 * (size_t)SmallFmt<T>::WBUF;
+    using F = SmallFmt<T>;
+    size_t b = (size_t)F::NXB * SXB + (size_t)F::NXB * SDX * 4 + (size_t)F::NWB * F::WBUF;
     if (T == IQ2_XXS || T == IQ3_S) b += sizeof(IqTables);
     return b;
 }
@@ -481,7 +542,8 @@ static hipError_t gemm_small_t(const GemmLaunch& g, hipStream_t s) {
     const int gno = g.pair ? SN / 2 : SN;
     const long long total = (long long)((g.rows + gno - 1) / gno) * g.n_tiles;
     if (total >= (1ll << 31)) return hipErrorInvalidValue;
-    const long long grid = std::max<long long>(std::min<long long>(total, ncu), 1);  // persistent: one block per CU
+    const long long fit = SmallFmt<T>::TWO ? 2 * ncu : ncu;  // persistent blocks: the ones resident at once
+    const long long grid = std::max<long long>(std::min<long long>(total, fit), 1);
     gemm_small_kernel<T><<<dim3((unsigned)grid), 64 * SW, smem, s>>>(a);
     return hipGetLastError();
 }

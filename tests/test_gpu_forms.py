@@ -58,8 +58,8 @@ def test_dense_gemm_few_positions(hip, ty, n, rows, cols):
 
 
 # tile lists of few positions: gathered gate/up and down rows on both sides of the dispatch lines of each kind of type
-@pytest.mark.parametrize("ty", [ggml.Q2_K, ggml.Q5_K, ggml.Q6_K, ggml.IQ4_XS])
-@pytest.mark.parametrize("t,cols", [(3, 512), (32, 2048), (33, 2048), (128, 1536), (129, 256)])
+@pytest.mark.parametrize("ty", [ggml.Q2_K, ggml.Q3_K, ggml.Q5_K, ggml.Q6_K, ggml.IQ4_XS, ggml.IQ2_XXS])
+@pytest.mark.parametrize("t,cols", [(3, 512), (32, 2048), (33, 2048), (48, 768), (49, 512), (128, 1536), (129, 256)])
 def test_grouped_gemm_few_positions(hip, ty, t, cols):
     """The 64-position tile list's GEMMs (SMALL_TILES) give the bits of the plain forms over the same tiles: the
     paired gate/up, a gathered store, and the rows of X in order (as a down GEMM reads them)."""
