@@ -79,9 +79,13 @@ __device__ __forceinline__ int neg_bytes(uint32_t g, uint32_t s) {
 // otherwise wait for every outstanding load before the first LDS read, and a load issued for a later super-block
 // could not overlap this one. The kernel waits for these loads itself (wait_loads) before the barrier that
 // publishes them. `lds` must be the same for every lane of the wave.
+// The compiler's hazard pass does not look into inline assembly, so each block keeps the wait states itself: one
+// between the write of M0 and the load that reads it (s_nop, or the copy of the base), and for a scalar base, which a
+// readfirstlane (VALU) may have written just before, the copy: a load may read an SGPR only five wait states after a VALU
+// instruction wrote it, but at once after a scalar one, and a scalar instruction may read it at once.
 __device__ __forceinline__ void load_lds16(uint64_t g, const void* lds) {
     const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(m0) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(m0) : "memory", "m0");
 }
 // The same from a wave-uniform 64-bit base plus a per-lane 32-bit byte offset (the base stays in scalar registers).
 __device__ __forceinline__ void load_lds16_so(uint64_t base, uint32_t off, const void* lds) {
@@ -89,14 +93,16 @@ __device__ __forceinline__ void load_lds16_so(uint64_t base, uint32_t off, const
     // readfirstlane returns int: widen through uint32_t, or bit 31 of the low half would spread into the high half
     const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32) |
                         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base);
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(sb), "s"(m0) : "memory", "m0");
+    uint64_t b;
+    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0" : "=&s"(b) : "v"(off), "s"(sb), "s"(m0) : "memory", "m0");
 }
 // 4 bytes per lane from a wave-uniform base plus a per-lane offset into LDS at lds + 4 * lane (global_load_lds_dword).
 __device__ __forceinline__ void load_lds4_so(uint64_t base, uint32_t off, const void* lds) {
     const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
     const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32) |
                         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base);
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(sb), "s"(m0) : "memory", "m0");
+    uint64_t b;
+    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dword %1, %0" : "=&s"(b) : "v"(off), "s"(sb), "s"(m0) : "memory", "m0");
 }
 // Block barrier after this wave's LDS operations complete, without waiting for its loads in flight (a
 // __syncthreads() fence would also wait for every outstanding vector memory operation).
