@@ -574,25 +574,16 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 
 // Eight softmax weights p (at most 8) times PF_SCALE as f16 hi and lo parts for the P V MFMA: hi = f16(p c), lo the exact
 // remainder p c - hi rounded likewise, both to nearest, so hi + lo carries each weight to 2^-22 of its value and the lo
-// parts stay normal f16 numbers for weights down to 2^-14. The mixed-precision multiply-adds scale, round and read the
-// f16 halves in place.
+// parts stay normal f16 numbers for weights down to 2^-14. Written so that the compiler selects the mixed-precision
+// multiply-adds, which scale, round and read the f16 halves in place (and keeps the wait states between them, the exps
+// before and the MFMAs after, as it could not for inline assembly).
 constexpr float PF_SCALE = 2048.0f;
 __device__ __forceinline__ void split_w8(const float* p, h8& hi, h8& lo) {
-    typedef float f2v __attribute__((ext_vector_type(2)));
-    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-    uint32_t hw[4], lw[4];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const float a = p[2 * e], b = p[2 * e + 1];
-        float ra, rb;
-        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(hw[e]) : "v"(a), "s"(PF_SCALE));
-        asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(hw[e]) : "v"(b), "s"(PF_SCALE));
-        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(ra) : "v"(a), "s"(PF_SCALE), "v"(hw[e]));
-        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(rb) : "v"(b), "s"(PF_SCALE), "v"(hw[e]));
-        lw[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2v){ra, rb}, h2v));
+    for (int e = 0; e < 8; e++) {
+        hi[e] = (_Float16)__builtin_fmaf(p[e], PF_SCALE, 0.0f);
+        lo[e] = (_Float16)__builtin_fmaf(p[e], PF_SCALE, -(float)hi[e]);
     }
-    hi = __builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3]));
-    lo = __builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3]));
 }
 // The larger of this lane's value and that of the lane 32 away.
 __device__ __forceinline__ float max_half(float v) {

@@ -83,3 +83,12 @@ def test_loads_into_lds_keep_their_wait_states(tmp_path):
         total += n
         assert not bad, (f, len(bad), bad[:4])
     assert total > 0
+
+
+def test_inline_assembly_computes_nothing():
+    """Arithmetic stays in forms that the compiler selects instructions for: it knows the wait states between a
+    transcendental result, a VALU write and an MFMA that reads it, but none of them for inline assembly."""
+    for f in sorted(os.listdir(build.CSRC)):
+        src = re.sub(r"//[^\n]*", "", open(os.path.join(build.CSRC, f)).read())
+        for body in re.findall(r"\basm\s*(?:volatile\s*)?\(\s*((?:\"[^\"]*\"\s*)+)", src):
+            assert not re.search(r"\bv_\w+", body), (f, body)
