@@ -5,10 +5,11 @@
 // adds nothing) and an optional gate (times sigmoid(qg[t, h 2 hd + hd + d])), as Model::attention
 // (src/model.rs:771-793) computes it.
 //
-// Prefill runs on f16 MFMA (v_mfma_f32_16x16x32_f16) without giving up f32 accuracy: q is split into f16 hi + lo
+// Prefill runs on f16 MFMA (v_mfma_f32_32x32x16_f16) without giving up f32 accuracy: q is split into f16 hi + lo
 // parts (q = hi + lo to 2^-22 relative) and so are the softmax weights, each product pair summed in f32, while K and V
-// are exact in f16 (the cache format). Both are scaled by powers of two first so that no part is a subnormal f16. Scores are computed transposed (S^T = K Q^T: keys on the MFMA rows), so the
-// softmax weights leave the score MFMA in exactly the register layout the P V MFMA takes as its B operand, and V sits
+// are exact in f16 (the cache format). Both are scaled by powers of two first, so that the lo parts of a query row's large
+// values and of weights down to 2^-17 are normal f16 numbers. Scores are computed transposed (S^T = K Q^T: keys on the
+// MFMA rows), so the softmax weights leave the score MFMA in exactly the register layout the P V MFMA takes as its B operand, and V sits
 // in LDS transposed ([dim][key]) for the A operand. Decode splits a token's positions over blocks (each serving all
 // query heads of one KV head) and merges the partial softmax sums in a second launch.
 #include <climits>
@@ -572,12 +573,14 @@ constexpr int PF_BK = 64;  // keys a tile (PfLayout's 64)
 constexpr int PF_Q = 32, PF_W = 4;  // query rows a wave; waves a block
 typedef float f16v __attribute__((ext_vector_type(16)));
 
-// Eight softmax weights p (at most 8) times PF_SCALE as f16 hi and lo parts for the P V MFMA: hi = f16(p c), lo the exact
+// Eight softmax weights p (at most 2) times PF_SCALE as f16 hi and lo parts for the P V MFMA: hi = f16(p c), lo the exact
 // remainder p c - hi rounded likewise, both to nearest, so hi + lo carries each weight to 2^-22 of its value and the lo
-// parts stay normal f16 numbers for weights down to 2^-14. Written so that the compiler selects the mixed-precision
-// multiply-adds, which scale, round and read the f16 halves in place (and keeps the wait states between them, the exps
-// before and the MFMAs after, as it could not for inline assembly).
-constexpr float PF_SCALE = 2048.0f;
+// parts stay normal f16 numbers for weights down to 2^-17. (2^14 is the largest scale that p = 2 leaves in f16, hence the
+// lag of 1: with a lag of 3 and 2^11, rows of weights around 2^-18 beside one of 1 were 1.4e-6 off, 7e-6 around 2^-20; the
+// time is the same.) Written so that the compiler selects the mixed-precision multiply-adds, which scale, round and read
+// the f16 halves in place (and keeps the wait states between them, the exps before and the MFMAs after, as it could not
+// for inline assembly).
+constexpr float PF_SCALE = 16384.0f;
 __device__ __forceinline__ void split_w8(const float* p, h8& hi, h8& lo) {
 #pragma unroll
     for (int e = 0; e < 8; e++) {
@@ -651,7 +654,7 @@ __global__ __launch_bounds__(64 * PF_W, 2) void attn_prefill_kernel(const float*
     for (int d = 0; d < DT; d++)
 #pragma unroll
         for (int i = 0; i < 16; i++) o[d][i] = 0.0f;
-    // m: a running maximum that may lag by 3, so the weights 2^(s - m) are at most 8; l: this lane's share of their sum
+    // m: a running maximum that may lag by 1, so the weights 2^(s - m) are at most 2; l: this lane's share of their sum
     float m = -INFINITY, l = 0.0f;
     const int qpos = pos0 + row;  // the lane's query position
     // K tile [key][dim] and V tile transposed [dim][key]; K chunk i = tid + NTH u of a tile: key i / ND, dims 8 (i % ND) ..;
@@ -725,12 +728,12 @@ __global__ __launch_bounds__(64 * PF_W, 2) void attn_prefill_kernel(const float*
 #pragma unroll
             for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[mt][i]);
         mx = max_half(mx);
-        // m follows the maximum only when a weight of the column would pass 8: the accumulators are rescaled in the first
+        // m follows the maximum only when a weight of the column would pass 2: the accumulators are rescaled in the first
         // tiles and hardly ever after them. (Column by column: a row's bits do not depend on the rows beside it, so not on
         // how a prompt is cut into chunks.)
         const float mxs = mx * usc;  // (a positive factor keeps the order)
-        if (__ballot(mxs > m + 3.0f)) {
-            const float mnew = mxs > m + 3.0f ? mxs : m, alpha = m == -INFINITY ? 0.0f : exp2_hw(m - mnew);
+        if (__ballot(mxs > m + 1.0f)) {
+            const float mnew = mxs > m + 1.0f ? mxs : m, alpha = m == -INFINITY ? 0.0f : exp2_hw(m - mnew);
             l *= alpha;
 #pragma unroll
             for (int d = 0; d < DT; d++) o[d] *= alpha;

@@ -152,6 +152,32 @@ def test_attn_prefill_rows_and_chunks(hip, nh, nkv, hd, t, pos, win):
         assert np.array_equal(one.view(np.uint32), run([t // 3 + 1, t - t // 3 - 1]).view(np.uint32))
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("gap", [16, 18, 20])
+def test_attn_prefill_small_weights_beside_a_sink(hip, hd, gap):
+    """The first key takes weight 1 (and has value 0), every other 2^-gap .. 2^(1 - gap): the running maximum never lags, so
+    the small weights are as far below the split's scale as they can be. Scores are exact (one dimension, a scale of
+    1 / log2 e), so what is left is the split, at most half an f16 subnormal (2^-25) of weights scaled by 2^14, that is
+    2^(gap - 39) of a weight, and the exps (1 ulp) and float32 sums: 5e-7."""
+    nh, nkv, t, pos = 8, 4, 33, 1000
+    n, rng = pos + t, np.random.default_rng(gap)
+    q, k = np.zeros((t, nh * hd), np.float32), np.zeros((n, nkv * hd), np.float16)
+    v = normal((n, nkv * hd), seed=gap + 1).astype(np.float16)
+    q[:, ::hd] = 1.0
+    k[:, ::hd] = rng.uniform(0.0, 1.0, (n, nkv)).astype(np.float16)
+    k[0, ::hd], v[0] = gap, 0.0
+    scale = float(np.float32(1.0 / 1.44269504088896341))
+    step, out = up(hip, np.array([pos, 0], np.int32)), hip.alloc(t * nh * hd * 4)
+    hip.attn_prefill(up(hip, q), up(hip, k), up(hip, v), 0, out, step, t, nh, nkv, hd, scale)
+    got = hip.get(out, np.float32, t * nh * hd).reshape(t, nh, hd)
+    for i in (0, t - 1):
+        for h in range(nh):
+            g = h // (nh // nkv)
+            w = np.exp(k[:pos + i + 1, g * hd].astype(np.float64) * scale)
+            want = w @ v[:pos + i + 1, g * hd:(g + 1) * hd].astype(np.float64) / w.sum()
+            assert rel_l2(got[i, h], want) <= 2.0 ** (gap - 39) + 5e-7, (i, h)
+
+
 # one block up to 4096 pairs, three launches beyond
 @pytest.mark.parametrize("t,k,E,chunk", [(1, 1, 1, 64), (3, 2, 512, 64), (512, 8, 128, 64), (512, 8, 512, 256), (513, 8, 128, 64)])
 def test_moe_sort_forms(hip, t, k, E, chunk):
