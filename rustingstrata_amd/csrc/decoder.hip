@@ -471,22 +471,28 @@ hipError_t launch_gemv_f32(const float* w, int rows, int cols, const float* x, u
 // ---- f32-weight GEMM (gemm_dense of a float matrix): each output's dot runs over k in index order with a multiply
 // then an add, as Tensor::matvec's f32 iterator sum (src/weights.rs:29-37): the CPU's bits. That makes every output
 // one dependent chain of 2 cols instructions (a lone wave issues one in 5-6 cycles), so few outputs are bound by the
-// chain and many by the VALU (62 us for 4096 x 128 x 2048 at two instructions a term). Three forms by the number of
-// outputs, n rows (launch_gemm_f32); router of 128 x 2048, us a call, before (one form: 4 chains a lane, x and weights
-// through one LDS buffer whose loads each step waited for) and now: 27 tokens 72 -> 18, 512 72 -> 28, 1501 72 -> 39,
+// chain and many by the VALU (62 us for 4096 x 128 x 2048 at two instructions a term). Four forms by the work they leave a
+// CU (gemm_f32_form); router of 128 x 2048, us a call, before (one form: 4 chains a lane, x and weights
+// through one LDS buffer whose loads each step waited for) and now: 27 tokens 72 -> 18, 512 72 -> 29, 1501 72 -> 39,
 // 4096 77 -> 68. ----
 
 // A block of 4 waves takes 64 positions (a lane each) x 4 RW weight rows (RW chains a lane). x and the weight rows come
-// by direct global-to-LDS loads into a ring of GF_NB steps of 32 k (four steps in flight: one step's work is shorter
-// than a trip to memory), the registers of a group are read from it one group ahead. x sits as [position][32 k] with
-// 16-byte chunk c of position p at c ^ ((p / 2) & 7): the 16 lanes of a 16-byte read touch every bank once.
-constexpr int GF_M = 64, GF_K = 32, GF_NB = 6;  // positions a block; k of a step; steps of x in the LDS ring
+// by direct global-to-LDS loads into a ring of gf_nb steps of 32 k (three or four steps in flight: one step's work is
+// shorter than a trip to memory), the registers of a group are read from it one group ahead. x sits as [position][32 k]
+// with 16-byte chunk c of position p at c ^ ((p / 2) & 7): the 16 lanes of a 16-byte read touch every bank once.
+constexpr int GF_M = 64, GF_K = 32;  // positions a block; k of a step
+// Steps in the LDS ring: as many as leave three blocks a CU (512 x 2048, 1501 positions: six steps, two blocks a CU 119 us,
+// five steps, three blocks 90).
+constexpr int gf_nb(int rw) { return rw == 1 ? 6 : 5; }
+constexpr int gf_lds(int rw) { return gf_nb(rw) * (GF_M + 4 * rw) * GF_K * 4; }
+static_assert(3 * gf_lds(1) <= 160 * 1024 && 3 * gf_lds(2) <= 160 * 1024 && 3 * gf_lds(4) <= 160 * 1024, "three blocks a CU");
 template <int RW>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ w, int rows, int cols,
                                                        const float* __restrict__ x, uint64_t x_stride, float* y,
                                                        uint64_t y_stride, int n, int act) {
     constexpr int GK = 32 / RW, GS = GF_K / GK;  // k of a register group; groups a step
     constexpr int NL = GF_M * GF_K * 4 / 1024 / 4;          // load instructions a wave and step
+    constexpr int GF_NB = gf_nb(RW);
     __shared__ __align__(16) float xs[GF_NB][GF_M * GF_K];
     __shared__ __align__(16) float ws[GF_NB][4 * RW * GF_K];
     const int m0 = blockIdx.x * GF_M, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -663,23 +669,48 @@ static void gemm_f32_t(const float* w, int rows, int cols, const float* x, uint6
     gemm_f32_kernel<RW><<<grid, dim3(256), 0, s>>>(w, rows, cols, x, x_stride, y, y_stride, n, act);
 }
 
+// The form of an F32 GEMM: 0 the quad form, else the ring form of that many rows a wave (1, 2, 4). Each form's cost in us
+// for 2048 columns, from what it leaves the fullest CU: the quad form by its waves a SIMD (2 positions x 16 rows each: 18 us
+// for one, 28-31 for two, 39 / 51 / 133 / 196 for 3 / 4 / 9 / 16), a ring form by its blocks of 64 positions x 4 RW rows, three
+// of them a CU at a time (RW 1: 29 / 31 / 40 us for 1 / 2 / 3 blocks, 57 / 72 / 96 for 4 / 6 / 8; RW 2: 41 / 46, 85 / 109 /
+// 142; RW 4: 59 / 68 / 90, 128 for 4, 213 for 8). Counting outputs alone gave a tall matrix of few positions to the ring
+// form with most lanes idle: 5 positions of 16384 x 2048 176 us, in the quad form 56.
+int gemm_f32_form(int n, int rows, int ncu) {
+    auto cdiv = [](long long a, long long b) { return (a + b - 1) / b; };
+    const long long r = cdiv(cdiv(n, 2) * cdiv(rows, 16), 4ll * ncu);
+    long long best = r == 1 ? 18 : r == 2 ? 29 : 13 * r + 4;
+    int form = 0;
+    constexpr int RW[3] = {1, 2, 4};
+    constexpr int COST[3][5] = {{29, 31, 36, 21, 26}, {41, 46, 54, 31, 38}, {59, 68, 88, 32, 40}};
+    for (int i = 0; i < 3; i++) {
+        const long long b = cdiv(cdiv(n, GF_M) * cdiv(rows, 4 * RW[i]), ncu);
+        const long long cost = b < 3 ? COST[i][b - 1] : COST[i][2] * (b / 3) + (b % 3 ? COST[i][2 + b % 3] : 0);
+        if (cost < best) {
+            best = cost;
+            form = RW[i];
+        }
+    }
+    return form;
+}
+
 hipError_t launch_gemm_f32(const float* w, int rows, int cols, const float* x, uint64_t x_stride, float* y,
                            uint64_t y_stride, int n, int act, hipStream_t s) {
     if (!rows || !n) return hipSuccess;
-    // by outputs (128 rows of 2048 columns, us; quad / RW 1 / 2 / 4): 256 positions 18 / 29 / 41 / 60, 512 28 / 29 / 41 /
-    // 61, 1024 51 / 31 / 41 / 61, 1501 73 / 39 / 45 / 61, 2048 96 / 56 / 46 / 61, 4096 186 / 93 / 89 / 68
+    static const int ncu = [] {
+        int dev = 0, v = 0;
+        return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
+    }();
     // (the ring's loads into LDS take 16-byte aligned weight rows, the quad form any float's address)
-    const long long outs = (long long)n * rows;
-    if (outs <= 65536 || (uintptr_t)w % 16) {
+    switch ((uintptr_t)w % 16 ? 0 : gemm_f32_form(n, rows, ncu)) {
+    case 0: {
         constexpr int P = 2, U = 8;
         const dim3 grid((unsigned)((n + 4 * P - 1) / (4 * P)), (unsigned)((rows + 15) / 16));
         gemm_f32_quad_kernel<P, U><<<grid, dim3(256), 0, s>>>(w, rows, cols, x, x_stride, y, y_stride, n, act);
-    } else if (outs <= 196608) {
-        gemm_f32_t<1>(w, rows, cols, x, x_stride, y, y_stride, n, act, s);
-    } else if (outs <= 262144) {
-        gemm_f32_t<2>(w, rows, cols, x, x_stride, y, y_stride, n, act, s);
-    } else {
-        gemm_f32_t<4>(w, rows, cols, x, x_stride, y, y_stride, n, act, s);
+        break;
+    }
+    case 1: gemm_f32_t<1>(w, rows, cols, x, x_stride, y, y_stride, n, act, s); break;
+    case 2: gemm_f32_t<2>(w, rows, cols, x, x_stride, y, y_stride, n, act, s); break;
+    default: gemm_f32_t<4>(w, rows, cols, x, x_stride, y, y_stride, n, act, s); break;
     }
     return hipGetLastError();
 }

@@ -16,11 +16,11 @@ def up(hip, a):
     return hip.upload(np.ascontiguousarray(a))
 
 
-# outputs n * rows: the quad form up to 65536, then 1, 2 and 4 rows a wave (lines at 196608 and 262144)
+# the quad form, and the ring form of 1, 2 and 4 rows a wave (1536, 1537 and 777 positions; rings of 6 and 5 steps of 32 columns)
 @pytest.mark.parametrize("n,rows,cols,off", [
     (1, 1, 4, 0), (5, 17, 36, 0), (8, 128, 256, 0), (63, 130, 100, 0), (512, 128, 516, 0), (513, 128, 516, 0),
     (600, 129, 28, 4), (1536, 128, 132, 0), (1537, 128, 100, 0), (2048, 128, 32, 0), (2049, 128, 164, 0),
-    (777, 515, 12, 0)])
+    (777, 515, 12, 0), (777, 515, 228, 0), (1501, 509, 292, 0), (5, 16385, 164, 0)])
 def test_f32_gemm_forms_are_the_sequential_sum(hip, n, rows, cols, off):
     """gemm_dense of a float matrix: every form gives the index-order float32 sum bit for bit (np.add over the columns
     one by one), for ragged rows, positions and columns, and for weights that are only float-aligned."""
