@@ -70,9 +70,15 @@ struct GemvArgs {
 };
 
 // LDS layout of gemv_kernel: [IqTables (IQ types)][x int8][x scales, f32][x sums, int32][weight tile], each section
-// rounded up to 16 bytes. Every 256-value super-block of x takes gxb bytes, gxd scales and gxs sums, one 16-byte chunk or
-// word more than its values where the LDS has room: the lanes of a wave read different super-blocks at once, which
-// without the padding all lie in the same banks (151936 x 2048 Q8_0, 3 inputs: 138 -> 100 us).
+// rounded up to 16 bytes. Every 256-value super-block of x takes gxb bytes, gxd scales and gxs sums: one 16-byte chunk or
+// word more than its values where gemv_pads says so. The lanes of a wave read different super-blocks at once, which
+// without the padding all lie in the same banks (151936 x 2048 Q8_0, 3 inputs: 138 -> 100 us). One input of Q6_K stays
+// without, in constants (1024 x 20480: 21.7 us, 25.4 with strides from the arguments, padded or not).
+template <int T, int NT> struct GemvX {
+    static constexpr bool PADS = !(T == Q6_K && NT == 1);
+    int b, d, s;  // bytes, scales, sums a super-block
+    __device__ explicit GemvX(const GemvArgs& a) : b(PADS ? a.gxb : 256), d(PADS ? a.gxd : 8), s(PADS ? a.gxs : 16) {}
+};
 __host__ __device__ constexpr uint32_t up16(uint32_t v) { return (v + 15) & ~15u; }
 
 // Sum over the g lanes of each aligned lane group (g a power of two <= 64).
@@ -135,12 +141,13 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
     IqTables* tab = (IqTables*)p;
     if constexpr (IQ) { load_iq_tables(tab); p += up16(sizeof(IqTables)); }
     const int nsb = (cols + 255) >> 8;
+    const GemvX<T, NT> gx(a);
     int8_t* sx = (int8_t*)p;
-    p += up16(NT * nsb * a.gxb);
+    p += up16(NT * nsb * gx.b);
     float* sd = (float*)p;
-    p += up16(NT * nsb * a.gxd * 4);
+    p += up16(NT * nsb * gx.d * 4);
     int* ss = (int*)p;
-    p += up16(NT * nsb * a.gxs * 4);
+    p += up16(NT * nsb * gx.s * 4);
     uint8_t* tile = p;
 
     // Tiles: t -> (z, slot, row tile); block b takes tiles b, b + grid, ... and prefetches the next one into
@@ -198,12 +205,12 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
             for (int c = tid; c < NT * cols / 16; c += GEMV_THREADS) {
                 const int u = c / (cols / 16), j = c % (cols / 16);
                 const v4u q = *gptr<v4u>((uint64_t)(a.xq + (uint64_t)(sp.xrow + u) * cols + 16 * j));
-                *(v4u*)(sx + (u * nsb + (j >> 4)) * a.gxb + 16 * (j & 15)) = q;
-                ss[(u * nsb + (j >> 4)) * a.gxs + (j & 15)] = sdot4((int)q.x, 0x01010101, sdot4((int)q.y, 0x01010101, sdot4((int)q.z, 0x01010101, sdot4((int)q.w, 0x01010101, 0))));
+                *(v4u*)(sx + __umul24(u * nsb + (j >> 4), gx.b) + 16 * (j & 15)) = q;
+                ss[__umul24(u * nsb + (j >> 4), gx.s) + (j & 15)] = sdot4((int)q.x, 0x01010101, sdot4((int)q.y, 0x01010101, sdot4((int)q.z, 0x01010101, sdot4((int)q.w, 0x01010101, 0))));
             }
             for (int c = tid; c < NT * cols / 32; c += GEMV_THREADS) {
                 const int u = c / (cols / 32), j = c % (cols / 32);
-                sd[(u * nsb + (j >> 3)) * a.gxd + (j & 7)] = *gptr<float>((uint64_t)(a.xd + (uint64_t)(sp.xrow + u) * (cols / 32) + j));
+                sd[__umul24(u * nsb + (j >> 3), gx.d) + (j & 7)] = *gptr<float>((uint64_t)(a.xd + (uint64_t)(sp.xrow + u) * (cols / 32) + j));
             }
             cur_xrow = sp.xrow;
         }
@@ -236,7 +243,8 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
                     const uint8_t* rowp = tile + (cs.beg - cs.g0) + (uint64_t)rr * a.rb;
 #pragma unroll
                     for (int u = 0; u < NT; u++) {
-                        const XLds xv{sx + (u * nsb + sb) * a.gxb, sd + (u * nsb + sb) * a.gxd, ss + (u * nsb + sb) * a.gxs};
+                        const int b = u * nsb + sb;
+                        const XLds xv{sx + __umul24(b, gx.b), sd + __umul24(b, gx.d), ss + __umul24(b, gx.s)};
                         const int nv = min(256, cols - 256 * sb);
                         f[u] = Q32 ? sb_dot_q32<T>(rowp + sb * SBB, xv, tab, nv) : sb_dot_q8k<T>(rowp + sb * SBB, xv, tab, nv);
                     }
@@ -861,6 +869,26 @@ static hipError_t gemv_t(const GemvArgs& a, long long grid, size_t smem, hipStre
     return a.per32 ? gemv_m<T, true>(a, grid, smem, s) : gemv_m<T, false>(a, grid, smem, s);
 }
 
+// LDS bytes of a gemv_kernel block.
+static size_t gemv_lds(int ty, int nt, int cols, bool pad) {
+    const uint32_t b = (uint32_t)nt * ((uint32_t)(cols + 255) / 256), p = pad;
+    return (size_t)(ty == IQ2_XXS || ty == IQ3_S ? up16(sizeof(IqTables)) : 0) + up16(b * (256 + 16 * p)) +
+           up16(b * (8 + p) * 4) + up16(b * (16 + p) * 4) + GEMV_TILE + 16;
+}
+// Whether gemv_kernel pads x's super-blocks: always where the same number of blocks fits a CU, or all tiles fit one round of
+// the padded ones. The second block of a CU is worth more (20480 columns, 2 inputs, Q8_0: 119 -> 203 us padded), and the
+// third for all but three types (1 input of 20480 columns, 20480 rows: Q5_K 250 -> 322, IQ4_XS 154 -> 200; but Q2_K 127 ->
+// 103; 3 of 6144, IQ2_XXS 148 -> 96, IQ3_S 210 -> 154), and for them where it saves a round of tiles (Q2_K 768 x 20480:
+// 14.4 -> 18.3).
+bool gemv_pads(int ty, int nt, int cols, long long tiles, int ncu) {
+    if (ty == Q6_K && nt == 1) return false;
+    constexpr size_t CU = 160 * 1024;
+    const size_t fit0 = CU / gemv_lds(ty, nt, cols, false), fit1 = CU / gemv_lds(ty, nt, cols, true);
+    if (fit1 == 0) return false;
+    if (fit1 == fit0 || tiles <= (long long)fit1 * ncu) return true;
+    return fit1 >= 2 && tiles > (long long)fit0 * ncu && (ty == Q2_K || ty == IQ2_XXS || ty == IQ3_S);
+}
+
 hipError_t launch_gemv(const GemvLaunch& g, hipStream_t s) {
     // Several inputs, or one of more columns than the register kernel takes: the MFMA form for few positions decodes a
     // weight once for all of them (151936 x 2048, 3 inputs, us: Q6_K 121 -> 62, Q4_K 75 -> 43, Q2_K 75 -> 31, IQ4_XS 76 ->
@@ -950,14 +978,9 @@ hipError_t launch_gemv(const GemvLaunch& g, hipStream_t s) {
         }
         return hipErrorInvalidValue;
     }
-    const uint32_t nsb = (uint32_t)(g.cols + 255) / 256;
-    auto lds = [&](int pad) {
-        a.gxb = 256 + 16 * pad; a.gxd = 8 + pad; a.gxs = 16 + pad;
-        return (size_t)(iq ? up16(sizeof(IqTables)) : 0) + up16(g.nt * nsb * a.gxb) + up16(g.nt * nsb * a.gxd * 4) +
-               up16(g.nt * nsb * a.gxs * 4) + GEMV_TILE + 16;
-    };
-    size_t smem = lds(1);
-    if (smem > 160 * 1024) smem = lds(0);
+    const bool pad = gemv_pads(g.ty, g.nt, g.cols, grid, ncu);
+    a.gxb = 256 + 16 * pad; a.gxd = 8 + pad; a.gxs = 16 + pad;
+    const size_t smem = gemv_lds(g.ty, g.nt, g.cols, pad);
     switch (g.ty) {
     case Q8_0: return gemv_t<Q8_0>(a, grid, smem, s);
     case Q2_K: return gemv_t<Q2_K>(a, grid, smem, s);

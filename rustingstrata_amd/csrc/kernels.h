@@ -63,6 +63,8 @@ struct GemvLaunch {
     float neps = 0.0f;
     int nck = 0;
 };
+// Whether gemv_kernel's x sits padded in LDS, for `tiles` tiles on ncu CUs.
+bool gemv_pads(int ty, int nt, int cols, long long tiles, int ncu);
 hipError_t launch_gemv(const GemvLaunch& g, hipStream_t s);
 // moe_down_combine as one launch: x[tk] += sum_j wh[tk k + j] W_{slots[j]} x_j (slots in order) + the shared expert,
 // x_j row tk k + j of xq. hipErrorNotSupported: a shape the fused layout does not take (cols not a multiple of 256,

@@ -4,7 +4,7 @@ import ctypes
 
 import pytest
 
-from rustingstrata_amd import backend
+from rustingstrata_amd import backend, ggml
 
 CUS = 256
 
@@ -32,3 +32,16 @@ def test_f32_gemm_form_of_any_size():
     for n in (1, 2, 63, 64, 65, 4097, 1 << 20, 1 << 30):
         for rows in (1, 3, 16, 17, 151936, 1 << 20, 1 << 30):
             assert f(n, rows, CUS) in (0, 1, 2, 4)
+
+
+@pytest.mark.parametrize("ty,nt,cols,tiles,pads", [
+    (ggml.Q8_0, 3, 2048, 40000, 1), (ggml.Q4_K, 4, 4096, 4096, 1),  # the same blocks a CU
+    (ggml.Q8_0, 2, 20480, 4096, 0), (ggml.Q2_K, 2, 20480, 4096, 0),  # one block a CU instead of two (119 us against 203)
+    (ggml.Q8_0, 1, 20480, 4096, 0), (ggml.Q5_K, 1, 20480, 20480, 0),  # two instead of three (51 against 60)
+    (ggml.Q2_K, 1, 20480, 6000, 1), (ggml.IQ3_S, 3, 6144, 5000, 1),   # worth it for these
+    (ggml.Q2_K, 1, 20480, 768, 0), (ggml.Q5_K, 1, 20480, 512, 1),     # a round of tiles
+    (ggml.Q6_K, 1, 18432, 512, 0)])
+def test_gemv_padding(ty, nt, cols, tiles, pads):
+    f = rule("_ZN6strata9gemv_padsEiiixi", ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_longlong, ctypes.c_int)
+    f.restype = ctypes.c_bool
+    assert f(ty, nt, cols, tiles, CUS) == bool(pads)
