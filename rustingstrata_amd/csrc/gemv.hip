@@ -889,12 +889,24 @@ bool gemv_pads(int ty, int nt, int cols, long long tiles, int ncu) {
     return fit1 >= 2 && tiles > (long long)fit0 * ncu && (ty == Q2_K || ty == IQ2_XXS || ty == IQ3_S);
 }
 
+// Whether several inputs, or one of more columns than the register kernel takes, go to the MFMA form for few positions,
+// which decodes a weight once for all of them (151936 x 2048, 3 inputs, us: Q6_K 121 -> 62, Q4_K 75 -> 43, Q2_K 75 -> 31,
+// IQ4_XS 76 -> 44; 2048 x 2048: Q6_K 11.8 -> 5.4, Q4_K 8.6 -> 4.6; 2 inputs of 4096 x 14336: Q6_K 48 -> 21). Its block takes
+// 16 rows and walks their super-blocks 8 at a time, so long rows have to fill its CUs, the more of them the fewer inputs
+// share a decode; gemv_kernel -> this form, us: 1 input of 20480 columns, 512 rows Q6_K 14.4 -> 28.9, Q4_K 13.5 -> 20, 1024
+// rows 21.7 -> 29.4, 20.3 -> 20.7, 2048 rows 36 -> 29.5, 24 -> 20.4 (Q3_K 27 -> 29.4, 4096 rows 37 -> 30); 2 inputs of 14336:
+// 512 rows Q6_K 16.4 -> 22.2, Q4_K 15.3 -> 16.6, 1000 rows 25 -> 22, 23 -> 17; of 8192: 768 rows 4% longer, 896 rows 26%
+// shorter (mean of the types); 3 of 28672: 256 rows 11% longer, 512 rows 26% shorter. Q8_0, per-32 numerics, paired and
+// routed forms never (launch_gemv_few).
+bool gemv_takes_few(int ty, int nt, int rows, int cols) {
+    if (nt > 1 && gemv_lds(ty, nt, cols, false) > 160 * 1024) return true;  // (more x than gemv_kernel holds)
+    if (nt == 1) return cols > GEMV1_MAX_COLS && rows >= (ty == Q3_K || ty == IQ2_XXS ? 4096 : 2048);
+    if (nt == 2) return cols < 3072 || rows > (cols < 12288 ? 768 : 512);
+    return nt > 3 || cols <= 24576 || rows > 256;
+}
+
 hipError_t launch_gemv(const GemvLaunch& g, hipStream_t s) {
-    // Several inputs, or one of more columns than the register kernel takes: the MFMA form for few positions decodes a
-    // weight once for all of them (151936 x 2048, 3 inputs, us: Q6_K 121 -> 62, Q4_K 75 -> 43, Q2_K 75 -> 31, IQ4_XS 76 ->
-    // 44; 2048 x 2048: Q6_K 11.8 -> 5.4, Q4_K 8.6 -> 4.6; 2 inputs of 4096 x 14336: Q6_K 48 -> 21). Q8_0, per-32
-    // numerics, paired and routed forms stay here.
-    if (g.nt > 1 || (g.cols > GEMV1_MAX_COLS && g.xq)) {
+    if (gemv_takes_few(g.ty, g.nt, g.rows, g.cols)) {
         const hipError_t e = launch_gemv_few(g, s);
         if (e != hipErrorNotSupported) return e;
     }

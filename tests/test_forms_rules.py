@@ -45,3 +45,19 @@ def test_gemv_padding(ty, nt, cols, tiles, pads):
     f = rule("_ZN6strata9gemv_padsEiiixi", ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_longlong, ctypes.c_int)
     f.restype = ctypes.c_bool
     assert f(ty, nt, cols, tiles, CUS) == bool(pads)
+
+
+@pytest.mark.parametrize("ty,nt,rows,cols,few", [
+    # one input of more columns than the register kernel takes: from 2048 rows (512 rows of Q6_K 14 us against 29)
+    (ggml.Q6_K, 1, 4096, 4096, 0), (ggml.Q6_K, 1, 512, 20480, 0), (ggml.Q4_K, 1, 2048, 20480, 1), (ggml.Q3_K, 1, 2048, 20480, 0),
+    (ggml.Q3_K, 1, 4096, 20480, 1),
+    # two: not few long rows
+    (ggml.Q6_K, 2, 64, 2048, 1), (ggml.Q6_K, 2, 512, 8192, 0), (ggml.Q6_K, 2, 1000, 8192, 1), (ggml.Q6_K, 2, 512, 14336, 0),
+    (ggml.Q6_K, 2, 640, 14336, 1),
+    (ggml.Q4_K, 3, 256, 28672, 0), (ggml.Q4_K, 3, 512, 28672, 1), (ggml.Q4_K, 4, 64, 28672, 1),
+    # more x than LDS holds otherwise
+    (ggml.Q2_K, 2, 64, 71680, 1), (ggml.Q2_K, 3, 64, 40960, 1)])
+def test_gemv_of_few_positions(ty, nt, rows, cols, few):
+    f = rule("_ZN6strata14gemv_takes_fewEiiii", ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int)
+    f.restype = ctypes.c_bool
+    assert f(ty, nt, rows, cols) == bool(few)

@@ -88,7 +88,8 @@ def test_grouped_gemm_few_positions(hip, ty, t, cols):
 
 
 @pytest.mark.parametrize("ty", ggml.TYPES)
-@pytest.mark.parametrize("rows,cols", [(3, 256), (33, 2304), (4097, 512), (20500, 256), (40, 20480)])
+@pytest.mark.parametrize("rows,cols", [(3, 256), (33, 2304), (4097, 512), (20500, 256), (40, 20480), (512, 12288), (513, 12288),
+                                       (2048, 16640)])
 def test_gemvn_few_positions_is_gemv(hip, ty, rows, cols):
     """2 to 4 inputs (and two matrices, gemvq2) give gemv's bits per input, under both numerics, whatever form takes
     them; rows over the 16384 columns of the register kernel against the CPU dots."""
