@@ -556,9 +556,7 @@ int strata_gemvq2(strata_ctx* c, const strata_tensor* a, const strata_tensor* b,
     if (a->rows > (1u << 30) || b->rows > (1u << 30)) return set_error("gemvq2: too many rows");
     if (check_gemv_cols(a->ty, a->cols, false) || check_align(a->ty, a->ptr, "gemvq2") || check_align(b->ty, b->ptr, "gemvq2")) return -1;
     if (!xq && nt > 1 && quant_into_scratch(c, x, x_stride, a->cols, nt, &xq)) return -1;
-    // several inputs: the form that serves them (launch_gemv) takes one matrix a launch, and two of its launches take
-    // less time than the paired one (6144 x 2048 Q6_K, 3 inputs: 11.6 us for one matrix paired or not, 7.1 there)
-    if (nt > 1 && a->ty != Q8_0 && c->numerics == STRATA_NUM_Q8K) {
+    if (c->numerics == STRATA_NUM_Q8K && gemvq2_splits(a->ty, (int)nt, (int)a->rows, (int)a->cols)) {
         if (strata_gemvq(c, a, x, x_stride, xq, ya, a->rows, nt)) return -1;
         return strata_gemvq(c, b, x, x_stride, xq, yb, b->rows, nt);
     }

@@ -905,6 +905,18 @@ bool gemv_takes_few(int ty, int nt, int rows, int cols) {
     return nt > 3 || cols <= 24576 || rows > 256;
 }
 
+// Whether gemvq2 of nt inputs is two launches, which may take the MFMA form for few positions, instead of gemv_kernel's one
+// over both matrices. One launch costs less where the matrices are small, or rows short and inputs few (one -> two, us:
+// 2 inputs of 6144 x 2048, Q6_K 11.3 -> 17, Q4_K 9.7 -> 13.4; mean of the types: 3 of 4096 x 4096 16% longer, 4 of 256 x 768
+// 17%, of 1024 x 4096 10%), two where the decode for every input outweighs it (2 of 8192 x 6144 26% shorter, 4096 x 11008
+// 50%; 3 of 1024 x 6144 13%; 4 of 512 x 2048 15%, 512 x 6144 25%).
+bool gemvq2_splits(int ty, int nt, int rows, int cols) {
+    if (ty == Q8_0 || nt < 2) return false;
+    if (nt == 2) return rows >= 4096 && cols >= 6144;
+    if (nt == 3) return rows >= 512 && cols >= 6144;
+    return cols >= 11008 || (rows >= 512 && (cols <= 2048 || cols >= 6144));
+}
+
 hipError_t launch_gemv(const GemvLaunch& g, hipStream_t s) {
     if (gemv_takes_few(g.ty, g.nt, g.rows, g.cols)) {
         const hipError_t e = launch_gemv_few(g, s);

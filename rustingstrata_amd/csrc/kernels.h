@@ -65,6 +65,8 @@ struct GemvLaunch {
 };
 // Whether a dense GEMV of nt inputs goes to the MFMA form for few positions.
 bool gemv_takes_few(int ty, int nt, int rows, int cols);
+// Whether two matrices of that type and shape and nt inputs are two launches.
+bool gemvq2_splits(int ty, int nt, int rows, int cols);
 // Whether gemv_kernel's x sits padded in LDS, for `tiles` tiles on ncu CUs.
 bool gemv_pads(int ty, int nt, int cols, long long tiles, int ncu);
 hipError_t launch_gemv(const GemvLaunch& g, hipStream_t s);

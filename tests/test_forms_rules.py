@@ -61,3 +61,14 @@ def test_gemv_of_few_positions(ty, nt, rows, cols, few):
     f = rule("_ZN6strata14gemv_takes_fewEiiii", ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int)
     f.restype = ctypes.c_bool
     assert f(ty, nt, rows, cols) == bool(few)
+
+
+@pytest.mark.parametrize("ty,nt,rows,cols,splits", [
+    (ggml.Q6_K, 1, 6144, 2048, 0), (ggml.Q8_0, 4, 6144, 2048, 0),
+    (ggml.Q6_K, 2, 6144, 2048, 0), (ggml.Q4_K, 2, 512, 4096, 0), (ggml.Q4_K, 2, 8192, 6144, 1),  # (11.3 us against 17)
+    (ggml.Q6_K, 3, 4096, 4096, 0), (ggml.Q4_K, 3, 1024, 6144, 1),
+    (ggml.Q6_K, 4, 256, 768, 0), (ggml.Q6_K, 4, 512, 2048, 1), (ggml.Q6_K, 4, 1024, 4096, 0), (ggml.Q6_K, 4, 256, 14336, 1)])
+def test_gemvq2_split(ty, nt, rows, cols, splits):
+    f = rule("_ZN6strata13gemvq2_splitsEiiii", ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int)
+    f.restype = ctypes.c_bool
+    assert f(ty, nt, rows, cols) == bool(splits)
