@@ -34,6 +34,8 @@ struct GemmLaunch {
 hipError_t launch_gemm(const GemmLaunch& g, hipStream_t s);
 // The form for few positions (gemm_few.hip): whether a GEMM takes it, and its launch.
 bool gemm_few_takes(const GemmLaunch& g);
+// The same of a tile list with SMALL_TILES: n_tiles slots, n_x rows of X that the tiles gather from or hold in order.
+bool gemm_few_takes_tiles(int ty, int rows, int cols, int n_tiles, bool gathered, int n_x);
 hipError_t launch_gemm_few(const GemmLaunch& g, hipStream_t s);
 // A GEMV of several pre-quantized inputs (one matrix, Q8_K numerics) through that form: the same bits;
 // hipErrorNotSupported where it does not apply.

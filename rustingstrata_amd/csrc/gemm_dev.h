@@ -40,6 +40,7 @@ struct GemmArgs {
     int64_t w2;           // pair: byte offset of the second matrix
     int dense_p;          // dense: positions per tile (GM, or less to give every CU an item)
     int bal;              // tile lists: an item's fixed cost in 16-position tiles, 0..47 (< 0: split by count)
+    int few_cs;           // gemm_few_kernel: an item takes every (1 << few_cs)-th chunk of its tile
 };
 
 // ---- the order of a tile list's items ----

@@ -38,30 +38,48 @@ constexpr int FPP = FPM + 4;  // floats of a term row (16-byte pad: rows start i
 // against 16.1 a wave an item (Q4_K 15.7 / 20.1), 256 of 2048 x 2048 22.2 / 16.2 (23.2 / 20.5).
 constexpr long long FEW_DENSE_BLOCK_ITEMS = 1280, FEW_DENSE_ITEMS = 2048;
 long long few_dense_items(int rows, int n) { return (long long)((rows + 15) / 16) * ((n + FPM - 1) / FPM); }
-// Tile lists with SMALL_TILES, 128 experts, top 8, 2048 x 768: gate/up by the tokens gathered from (27 / 100 / 200
-// tokens): Q3_K 81 -> 65 / 120 -> 110 / 122 -> 138 (128 tokens: 121 -> 121), IQ2_XXS 69 -> 57 / 103 -> 95 / 105 -> 119
-// (128: 104 -> 103), Q2_K 48 -> 42 / 67 -> 67 / 69 -> 92 (48: 57 -> 55, 64: 58 -> 62); the scale-after types, whose close
-// is heavier per tile, only up to 32 tokens: Q5_K 64 -> 53 / 94 -> 103, Q4_K 59 -> 51 / 86 -> 94, IQ4_XS 72 -> 54 / 102
-// -> 98 (64 tokens: 82 -> 87). Down by the rows of X (216 / 512 / 800): Q3_K 43 -> 37 / 52 -> 51 / 57 -> 61, IQ2_XXS 46 ->
-// 38 / 58 -> 54 / 63 -> 64, Q2_K 27 -> 24 / 32 -> 35 / 35 -> 44 (384: 31 -> 31), Q6_K 50 -> 35 / - / 72 -> 61 (1600: 72
-// -> 62); IQ4_XS 40 -> 37 (320: 47 -> 42, 512: 50 -> 54), IQ3_S 47 -> 39; Q4_K 128: 25 -> 23, 216: 33 -> 37, Q5_K 27 ->
-// 24, 36 -> 38. At most 12 rows a tile slot: with fewer, fuller tiles every 16 positions would decode the weights again.
-int few_gathered(int ty) {
+// Tile lists with SMALL_TILES, gemm_small_kernel -> this form.
+// Gate/up, by the tokens gathered from (128 experts, top 8, 2048 x 768; us at 27 / 100 / 200 tokens): Q3_K 81 -> 65 / 120 ->
+// 110 / 122 -> 138, IQ2_XXS 69 -> 57 / 103 -> 95 / 105 -> 119, Q2_K 48 -> 42 / 67 -> 67 / 69 -> 92 (48: 57 -> 55, 64: 58 ->
+// 62); the scale-after types, whose close is heavier per tile, only up to 32 tokens: Q5_K 64 -> 53 / 94 -> 103, Q4_K 59 ->
+// 51 / 86 -> 94, IQ4_XS 72 -> 54 / 102 -> 98 (64 tokens: 82 -> 87). This form's time over the other's, for even and
+// Zipf-skewed loads, with 128 experts top 8 / 64 top 6 / 32 top 4 (1024 columns) / 8 top 2: Q3_K 100 tokens 0.92 1.02 / 0.92
+// 1.17 / 0.99 0.95 / 0.66 0.73, 128 tokens 0.92 1.19 / 1.03 1.24 / 0.98 0.88 / 0.77 0.91 (IQ2_XXS alike); Q6_K 64 tokens 0.79
+// 0.81 / 0.76 0.84 / 0.78 0.90 / 0.71 0.67, 100 tokens 0.79 0.88 / 0.77 0.95 / 1.08 1.05 / 0.72 0.79, 128 tokens 0.81 0.98 /
+// 0.87 1.00 / 1.09 0.91 / 0.84 0.99; 32 tokens, the others, at most 0.96.
+// Down, by the rows of X (128 experts; 216 / 512 / 800): Q3_K 43 -> 37 / 52 -> 51 / 57 -> 61, IQ2_XXS 46 -> 38 / 58 -> 54 /
+// 63 -> 64, Q2_K 27 -> 24 / 32 -> 35 / 35 -> 44 (384: 31 -> 31), Q6_K 50 -> 35 / - / 72 -> 61 (1600: 72 -> 62); IQ4_XS 40 ->
+// 37 (320: 47 -> 42, 512: 50 -> 54), IQ3_S 47 -> 39; Q4_K 128: 25 -> 23, 216: 33 -> 37, Q5_K 27 -> 24, 36 -> 38.
+// And by the rows a tile slot, because every 16 positions of a tile decode its weights again: over the other form's time, even
+// and skewed, at 3 rows an expert (128 experts / 64): Q4_K 0.87 1.03 / 0.90 1.09, IQ4_XS 0.71 0.89 / 0.74 0.93, at 4 and 4.5
+// IQ4_XS 0.74 1.10 / 0.77 1.17, IQ3_S 0.67 0.99 / 0.69 1.03, Q2_K 0.75 1.17 / 0.70 1.07, at 6 Q2_K 0.79 1.15 / 0.79 1.30, Q3_K
+// 0.77 0.98 / 0.75 1.10, Q6_K at 8 and 12 0.64 0.84 / 0.89 0.98. With less than an item a wave, where a tile's chunks run
+// side by side: 32 experts of 1024 x 512 at 6 / 8 / 12.5 rows an expert Q6_K 0.60 0.76 / 0.60 0.79 / 0.82 1.29, Q4_K 0.80 0.72
+// / 0.82 0.99 / 1.03 1.73 (one after the other, 0.57 1.15 and 0.77 1.40 at 6); 8 experts of 2048 x 1024 at 12 / 16: Q6_K
+// 0.59 0.59 / 0.59 0.81, Q4_K 0.89 0.90 / 0.89 1.01, IQ4_XS 0.86 0.86 / 0.87 1.05.
+int few_gathered(int ty, int cols) {
     switch (ty) {
-    case Q3_K: case Q6_K: case IQ2_XXS: return 128;
+    case Q6_K: return cols < 1536 ? 64 : 128;
+    case Q3_K: case IQ2_XXS: return 100;
     case Q2_K: return 48;
     default: return 32;
     }
 }
-int few_rows(int ty) {
+// Most rows of X, and most quarter rows a tile slot where every wave has an item.
+struct FewRows {
+    int rows, slot4;
+};
+FewRows few_rows(int ty) {
     switch (ty) {
-    case Q6_K: return 1024;
-    case Q3_K: case IQ2_XXS: return 512;
-    case Q2_K: return 384;
-    case IQ3_S: case IQ4_XS: return 320;
-    default: return 128;
+    case Q6_K: return {1024, 48};
+    case Q3_K: case IQ2_XXS: return {512, 26};
+    case Q2_K: return {384, 18};
+    case IQ3_S: return {320, 16};
+    case IQ4_XS: return {320, 12};
+    default: return {128, 10};
     }
 }
+constexpr int FEW_WAVES = 256 * 2 * FW;  // waves resident at once
 }  // namespace
 
 template <int T> struct FewFmt : GemmPlanes<T> {
@@ -91,7 +109,8 @@ __global__ __launch_bounds__(64 * FW, 4) void gemm_few_kernel(GemmArgs a) {
     const int cols = a.cols, nsb = cols / 256, l16 = lane & 15, kl = lane >> 4;
     const int ntiles = a.tiles ? (a.n_tiles_dev ? min(sload(a.n_tiles_dev), a.max_tiles) : a.max_tiles) : a.max_tiles;
     const bool pair = KSP && a.pair != 0;
-    const int nrb = (a.rows + 15) / 16, total = nrb * ntiles;
+    // an item is a tile's 16 rows and every (1 << cs)-th of its chunks of 16 positions, the first chunks' items first
+    const int nrb = (a.rows + 15) / 16, nit = nrb * ntiles, cs = KSP ? 0 : a.few_cs, total = nit << cs;
     // this wave's super-blocks s0, s0 + KS, .. of an item, of the second matrix (pair) for waves 4..7
     const int mat = pair ? wave >> 2 : 0, KS = !KSP ? 1 : pair ? 4 : 8, s0 = !KSP ? 0 : pair ? wave & 3 : wave;
     const uint64_t w2 = mat ? (uint64_t)a.w2 : 0;
@@ -99,28 +118,34 @@ __global__ __launch_bounds__(64 * FW, 4) void gemm_few_kernel(GemmArgs a) {
 
     struct Item {
         uint64_t w;
-        int m0, cnt, n0, rest;  // cnt 0: no item; rest: the tile's positions after this chunk
+        int m0, cnt, n0, rest;  // cnt 0: no item; rest > 0: the item has a chunk after this one
     };
     auto item_at = [&](int id, int pc) __attribute__((always_inline)) {
         Item it;
+        int c = pc << cs;
+        if (cs) {  // (at most 4 chunks side by side)
+            const int q = (id >= nit) + (id >= 2 * nit) + (id >= 3 * nit);
+            c += q;
+            id -= q * nit;
+        }
         const int tile = id / nrb;
         it.n0 = 16 * (id - tile * nrb);
         int cnt;
         if (a.tiles) {
             const uint64_t t0 = sload(a.tiles + 2 * tile), t1 = sload(a.tiles + 2 * tile + 1);
             it.w = t0;
-            it.m0 = (int)(uint32_t)t1 + FPM * pc;
-            cnt = min(256, (int)(t1 >> 32)) - FPM * pc;
+            it.m0 = (int)(uint32_t)t1 + FPM * c;
+            cnt = min(256, (int)(t1 >> 32)) - FPM * c;
         } else {
             it.w = (uint64_t)a.dense_w;
             it.m0 = FPM * tile;
             cnt = min(FPM, a.dense_n - it.m0);
         }
         it.cnt = max(0, min(FPM, cnt));
-        it.rest = cnt - it.cnt;
+        it.rest = cnt - (FPM << cs);
         return it;
     };
-    // the next chunk with positions: the next of the same tile, else the first of the next item that has any
+    // the next chunk with positions: the next of the same item, else the first of the next item that has any
     auto next_item = [&](int& id, int& pc, const Item& prev) __attribute__((always_inline)) {
         if (prev.rest > 0) return item_at(id, ++pc);
         Item it{0, 0, 0, 0, 0};
@@ -345,7 +370,7 @@ static hipError_t few_launch(const GemmArgs& a, hipStream_t s) {
         if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
         if (e != hipSuccess) return e;
     }
-    const long long total = (long long)((a.rows + 15) / 16) * a.max_tiles;
+    const long long total = ((long long)((a.rows + 15) / 16) * a.max_tiles) << a.few_cs;
     if (total >= (1ll << 31)) return hipErrorInvalidValue;
     const long long want = KSP ? total : (total + FW - 1) / FW;
     const long long grid = std::max<long long>(std::min<long long>(want, 2ll * ncu), 1);  // persistent: two blocks per CU
@@ -369,6 +394,8 @@ static hipError_t few_t(const GemmLaunch& g, hipStream_t s) {
         a.max_tiles = (g.dense_n + FPM - 1) / FPM;
         ksp = few_dense_items(g.rows, g.dense_n) <= FEW_DENSE_BLOCK_ITEMS;
     }
+    // with less than an item a wave, a tile's chunks side by side: the largest expert's would otherwise set the time
+    if (g.tiles && !ksp && (long long)((g.rows + 15) / 16) * g.n_tiles < FEW_WAVES) a.few_cs = 2;
     return ksp ? few_launch<T, true>(a, s) : few_launch<T, false>(a, s);
 }
 
@@ -385,12 +412,19 @@ hipError_t launch_gemv_few(const GemvLaunch& g, hipStream_t s) {
     return launch_gemm_few(m, s);
 }
 
+bool gemm_few_takes_tiles(int ty, int rows, int cols, int n_tiles, bool gathered, int n_x) {
+    const long long items = (long long)((rows + 15) / 16) * n_tiles;
+    if (ty == Q8_0 || items >= (1ll << 31)) return false;
+    if (gathered) return n_x <= few_gathered(ty, cols);
+    const FewRows f = few_rows(ty);
+    const int slot4 = items < FEW_WAVES / 2 ? 48 : items < FEW_WAVES ? 32 : f.slot4;
+    return n_x <= f.rows && 4ll * n_x <= (long long)slot4 * n_tiles;
+}
+
 bool gemm_few_takes(const GemmLaunch& g) {
     if (g.ty == Q8_0) return false;
     if (!g.tiles) return g.dense_n <= FPM || few_dense_items(g.rows, g.dense_n) <= FEW_DENSE_ITEMS;
-    if (!g.small || (long long)((g.rows + 15) / 16) * g.n_tiles >= (1ll << 31)) return false;
-    if (g.xrow) return g.n_x <= few_gathered(g.ty);
-    return g.n_x <= few_rows(g.ty) && g.n_x <= 12ll * g.n_tiles;
+    return g.small && gemm_few_takes_tiles(g.ty, g.rows, g.cols, g.n_tiles, g.xrow != nullptr, g.n_x);
 }
 
 hipError_t launch_gemm_few(const GemmLaunch& g, hipStream_t s) {

@@ -72,3 +72,23 @@ def test_gemvq2_split(ty, nt, rows, cols, splits):
     f = rule("_ZN6strata13gemvq2_splitsEiiii", ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int)
     f.restype = ctypes.c_bool
     assert f(ty, nt, rows, cols) == bool(splits)
+
+
+# (tile slots: 128 experts of 768 x 2048 and 2048 x 768, 64 of 1024 x 2048 and 2048 x 1024, 32 of 512 x 1024 and 1024 x 512, 8 of
+# 1024 x 2048 and 2048 x 1024)
+@pytest.mark.parametrize("ty,rows,cols,n_tiles,gathered,n_x,few", [
+    # gathered: by the tokens (128 tokens of Q3_K over 64 experts, skewed: 1.24 times the time)
+    (ggml.Q3_K, 1024, 2048, 73, 1, 100, 1), (ggml.Q3_K, 1024, 2048, 76, 1, 128, 0), (ggml.Q6_K, 768, 2048, 144, 1, 128, 1),
+    (ggml.Q6_K, 512, 1024, 38, 1, 100, 0), (ggml.Q4_K, 768, 2048, 132, 1, 33, 0), (ggml.Q8_0, 768, 2048, 132, 1, 8, 0),
+    # rows in order: by the rows, and by the rows a slot
+    (ggml.Q2_K, 2048, 768, 134, 0, 384, 1), (ggml.Q2_K, 2048, 1024, 70, 0, 384, 0), (ggml.Q2_K, 2048, 1024, 66, 0, 192, 1),
+    (ggml.IQ4_XS, 2048, 1024, 68, 0, 294, 0), (ggml.IQ4_XS, 2048, 768, 133, 0, 320, 1), (ggml.Q6_K, 2048, 1024, 76, 0, 768, 1),
+    (ggml.Q4_K, 2048, 768, 130, 0, 128, 1), (ggml.Q4_K, 2048, 768, 131, 0, 216, 0),
+    # less than an item, and than half an item, a wave
+    (ggml.IQ4_XS, 1024, 512, 36, 0, 256, 1), (ggml.Q6_K, 1024, 512, 38, 0, 400, 0), (ggml.Q4_K, 2048, 1024, 9, 0, 98, 1),
+    (ggml.Q4_K, 2048, 1024, 10, 0, 128, 0)])
+def test_tile_lists_of_few_positions(ty, rows, cols, n_tiles, gathered, n_x, few):
+    f = rule("_ZN6strata20gemm_few_takes_tilesEiiiibi", ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_bool,
+             ctypes.c_int)
+    f.restype = ctypes.c_bool
+    assert f(ty, rows, cols, n_tiles, bool(gathered), n_x) == bool(few)

@@ -87,6 +87,27 @@ def test_grouped_gemm_few_positions(hip, ty, t, cols):
         assert np.array_equal(a, b), i
 
 
+# (empty tiles: slots that keep the rows a slot under the rule's line)
+@pytest.mark.parametrize("ty", [ggml.Q2_K, ggml.Q3_K, ggml.IQ4_XS, ggml.IQ3_S])
+@pytest.mark.parametrize("sizes,rows", [([1, 16, 17, 63, 64, 65, 0, 2] + [0] * 21, 33), ([0] * 15 + [200] + [0] * 9, 64),
+                                        ([130, 3, 1] + [0] * 14, 2000), ([5] * 40, 1600)])
+def test_grouped_gemm_chunks_side_by_side(hip, ty, sizes, rows):
+    """Tile lists of less than an item a wave, whose tiles' chunks of 16 positions run side by side (and past 64 positions one
+    after the other again), against the plain form: the same bits, no row left out or written twice (act add)."""
+    cols, n = 512, sum(sizes)
+    st = ggml.row_bytes(ty, cols) * rows
+    w, x = up(hip, random_blocks(ty, rows * min(len(sizes), 8), cols, seed=ty)), up(hip, normal((n, cols), seed=n))
+    m0 = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    tiles = np.array([[int(w) + (i % 8) * st, int(m) | (c << 32)] for i, (m, c) in enumerate(zip(m0, sizes))], np.uint64)
+    tb, y, out = up(hip, tiles), hip.alloc(n * rows * 4), []
+    for flag in (0, S.SMALL_TILES):
+        hip.memset(y)
+        for act in (S.ACT_STORE, S.ACT_ADD):
+            hip.gemm(ty, rows, cols, tb, len(sizes), x, cols, n, 0, y, rows, act | flag)
+        out.append(hip.get(y, np.uint32, n * rows))
+    assert np.array_equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("ty", ggml.TYPES)
 @pytest.mark.parametrize("rows,cols", [(3, 256), (33, 2304), (4097, 512), (20500, 256), (40, 20480), (512, 12288), (513, 12288),
                                        (2048, 16640)])
