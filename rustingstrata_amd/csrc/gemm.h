@@ -41,6 +41,8 @@ hipError_t launch_gemm_few(const GemmLaunch& g, hipStream_t s);
 // hipErrorNotSupported where it does not apply.
 struct GemvLaunch;
 hipError_t launch_gemv_few(const GemvLaunch& g, hipStream_t s);
+// The Q8_0 GEMM's grid of 256-thread blocks for that many items.
+dim3 gemm_q8_0_grid(long long total);
 hipError_t launch_gemm_small(const GemmLaunch& g, hipStream_t s);
 // Positions of one GEMM block (a tile list's chunks of this size give every block a full tile).
 uint64_t gemm_block_positions();

@@ -647,6 +647,11 @@ __global__ __launch_bounds__(256, 3) void gemm_q8_0_kernel(GemmArgs a) {
     }
 }
 
+// The grid for `total` items: HIP takes fewer than 2^32 threads along x, so longer runs go on in slices along y.
+dim3 gemm_q8_0_grid(long long total) {
+    const long long x = std::min((total + NXCD - 1) / NXCD * NXCD, 1ll << 23);
+    return dim3((unsigned)x, (unsigned)((total + x - 1) / x));
+}
 static hipError_t gemm_q8_0(const GemmLaunch& g, hipStream_t s) {
     GemmArgs a{};
     a.tiles = g.tiles; a.n_tiles_dev = g.n_tiles_dev; a.dense_w = g.dense_w; a.dense_n = g.dense_n;
@@ -655,9 +660,8 @@ static hipError_t gemm_q8_0(const GemmLaunch& g, hipStream_t s) {
     a.rb = row_bytes(Q8_0, g.cols);
     a.max_tiles = g.tiles ? g.n_tiles : (g.dense_n + Q8_POS - 1) / Q8_POS;
     const long long total = (long long)((g.rows + Q8_ROWS - 1) / Q8_ROWS) * a.max_tiles;
-    const long long grid = std::min((total + NXCD - 1) / NXCD * NXCD, 1ll << 30), ny = (total + grid - 1) / std::max(grid, 1ll);
-    if (ny > 65535) return hipErrorInvalidValue;
-    gemm_q8_0_kernel<<<dim3((unsigned)grid, (unsigned)ny), 256, 0, s>>>(a);
+    if (total <= 0) return hipSuccess;
+    gemm_q8_0_kernel<<<gemm_q8_0_grid(total), 256, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -92,3 +92,15 @@ def test_tile_lists_of_few_positions(ty, rows, cols, n_tiles, gathered, n_x, few
              ctypes.c_int)
     f.restype = ctypes.c_bool
     assert f(ty, rows, cols, n_tiles, bool(gathered), n_x) == bool(few)
+
+
+@pytest.mark.parametrize("total", [1, 7, 8, 1000, 1 << 23, (1 << 23) + 1, 1 << 24, (1 << 24) + 8, (1 << 18) * 65535])
+def test_q8_0_grid(total):
+    """Every item has a block, and HIP takes the grid (fewer than 2^32 threads along x, 65536 blocks along y)."""
+    class Dim3(ctypes.Structure):
+        _fields_ = [("x", ctypes.c_uint), ("y", ctypes.c_uint), ("z", ctypes.c_uint)]
+    f = rule("_ZN6strata14gemm_q8_0_gridEx", ctypes.c_longlong)
+    f.restype = Dim3
+    g = f(total)
+    assert g.x % 8 == 0 and g.x * 256 < 1 << 32 and 0 < g.y < 1 << 16 and g.z == 1
+    assert g.x * g.y >= total

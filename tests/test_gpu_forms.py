@@ -57,6 +57,29 @@ def test_dense_gemm_few_positions(hip, ty, n, rows, cols):
     assert np.array_equal(hip.get(yb, np.float32, n * rows).reshape(n, rows), got + got)
 
 
+def test_q8_0_grid_in_slices(hip):
+    """More items than one slice of the grid holds (65535 tiles of one position x 129 row blocks): the items at the slices'
+    ends on every XCD, and the first and last ones, against the same rows of X as one dense GEMM."""
+    ty, rows, cols, nt = ggml.Q8_0, 64 * 129, 256, 65535
+    w, x = random_blocks(ty, rows, cols, seed=5), normal((5, cols), seed=6)
+    t, xb, y = hip.upload_tensor(ty, w), up(hip, x), hip.alloc(nt * rows * 4)
+    i = np.arange(nt, dtype=np.uint64)
+    tiles = up(hip, np.stack([np.full(nt, t.ptr, np.uint64), i | np.uint64(1 << 32)], axis=1))
+    xrow, yd = up(hip, (i % 5).astype(np.int32)), hip.alloc(5 * rows * 4)
+    hip.memset(y)
+    hip.gemm(ty, rows, cols, tiles, nt, xb, cols, 5, xrow, y, rows, S.ACT_STORE)
+    hip.gemm_dense(t, 5, xb, cols, yd, rows, S.ACT_STORE)
+    want = hip.get(yd, np.uint32, 5 * rows).reshape(5, rows)
+    total, per = 129 * nt, -(-129 * nt // 8)
+    assert total > 1 << 23
+    for xcd in range(8):
+        for at in (0, 1, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, per - 2, per - 1):
+            item = min(xcd * per + at, total - 1)
+            rb, tile = divmod(item, nt)
+            got = hip.get(y, np.uint32, 64, at=tile * rows + 64 * rb)
+            assert np.array_equal(got, want[tile % 5, 64 * rb:64 * rb + 64]), (xcd, at)
+
+
 # tile lists of few positions: gathered gate/up and down rows on both sides of the dispatch lines of each kind of type
 @pytest.mark.parametrize("ty", [ggml.Q2_K, ggml.Q3_K, ggml.Q5_K, ggml.Q6_K, ggml.IQ4_XS, ggml.IQ2_XXS])
 @pytest.mark.parametrize("t,cols", [(3, 512), (32, 2048), (33, 2048), (48, 768), (49, 512), (128, 1536), (129, 256)])
