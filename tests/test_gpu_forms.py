@@ -168,8 +168,10 @@ def test_gemvn_few_positions_is_gemv(hip, ty, rows, cols):
 @pytest.mark.parametrize("t,pos,win", [(1, 0, 0), (31, 63, 0), (33, 100, 0), (130, 1, 48), (257, 64, 64)])
 def test_attn_prefill_rows_and_chunks(hip, nh, nkv, hd, t, pos, win):
     """Rows at the edges of the 32-row tiles, the 64-key tiles and the window, per GQA group (heads and row tiles share a
-    block differently), against the f64 attention (float32 sums: 2e-5 of the row's norm); the same rows computed as
-    chunks of other sizes give the same bits. One query row is large, so that the running maximum jumps between tiles."""
+    block differently), against the f64 attention; the same rows computed as chunks of other sizes give the same bits. One
+    query row is large, so that the running maximum jumps between tiles. Tolerance: a float32 score s is off by 2^-24 |s| in
+    its sum and again in the exponent, which is the weight's relative error; the exps, the splits (2^-22) and the two sums add
+    eight times 2^-23 at most (8.8e-7 seen in ordinary rows, 8.9e-6 in the large one, whose scores reach 120)."""
     n = pos + t
     q, k, v = normal((t, nh * hd), seed=1), normal((n, nkv * hd), seed=2).astype(np.float16), normal((n, nkv * hd), seed=3).astype(np.float16)
     q[t // 2] *= 30.0
@@ -192,7 +194,7 @@ def test_attn_prefill_rows_and_chunks(hip, nh, nkv, hd, t, pos, win):
             kk, vv = (a[lo:pos + i + 1, g * hd:(g + 1) * hd].astype(np.float64) for a in (k, v))
             s = kk @ q[i, h * hd:(h + 1) * hd].astype(np.float64) / np.sqrt(hd)
             w = np.exp(s - s.max())
-            assert rel_l2(one[i, h], w @ vv / w.sum()) <= 2e-5, (i, h)
+            assert rel_l2(one[i, h], w @ vv / w.sum()) <= 2.0 ** -23 * (8 + np.abs(s).max()), (i, h)
     if t > 1:
         assert np.array_equal(one.view(np.uint32), run([t // 3 + 1, t - t // 3 - 1]).view(np.uint32))
 
@@ -221,6 +223,87 @@ def test_attn_prefill_small_weights_beside_a_sink(hip, hd, gap):
             w = np.exp(k[:pos + i + 1, g * hd].astype(np.float64) * scale)
             want = w @ v[:pos + i + 1, g * hd:(g + 1) * hd].astype(np.float64) / w.sum()
             assert rel_l2(got[i, h], want) <= 2.0 ** (gap - 39) + 5e-7, (i, h)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 8, 128), (8, 2, 64)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_attn_prefill_non_finite(hip, nh, nkv, hd, bad):
+    """A query row that is not finite spoils its own row of its head and no other; a key that is not a number spoils every row
+    that sees it (in the heads of its group) and no row before it; a value row's element its column from that key on, and in
+    no tile of 32 rows that ends before its tile of 64 keys (a masked weight is an exact 0, which a product with a value that
+    is not finite does not stay)."""
+    t, pos, j, d = 100, 60, 131, 5
+    n, G = pos + t, nh // nkv
+    q, k, v = normal((t, nh * hd), seed=1), normal((n, nkv * hd), seed=2).astype(np.float16), normal((n, nkv * hd), seed=3).astype(np.float16)
+    step, out = up(hip, np.array([pos, 0], np.int32)), hip.alloc(t * nh * hd * 4)
+
+    def run(q, k, v):
+        hip.attn_prefill(up(hip, q), up(hip, k), up(hip, v), 0, out, step, t, nh, nkv, hd, 1.0 / np.sqrt(hd))
+        return hip.get(out, np.float32, t * nh * hd).reshape(t, nh, hd)
+
+    def same(a, b):
+        return np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+    clean = run(q, k, v)
+    q1, k1, v1 = q.copy(), k.copy(), v.copy()
+    q1[40, 3 * hd + d] = bad
+    got = run(q1, k, v)
+    assert not np.isfinite(got[40, 3]).any()
+    got[40, 3] = clean[40, 3]
+    assert same(got, clean)
+    k1[j, hd + d] = np.nan
+    got = run(q, k1, v)
+    assert not np.isfinite(got[j - pos:, G:2 * G]).any() and same(got[:j - pos], clean[:j - pos])
+    got[:, G:2 * G] = clean[:, G:2 * G]
+    assert same(got, clean)
+    v1[j, hd + d] = bad
+    got = run(q, k, v1)
+    r = (j // 64 * 64 - pos) // 32 * 32
+    assert not np.isfinite(got[j - pos:, G:2 * G, d]).any() and same(got[:r], clean[:r])
+    got[:, G:2 * G, d] = clean[:, G:2 * G, d]
+    assert same(got, clean)
+
+
+@pytest.mark.parametrize("n,rows,cols", [(8, 128, 256), (1536, 128, 132), (1537, 128, 100), (777, 515, 228)])
+def test_f32_gemm_non_finite(hip, n, rows, cols):
+    """Infinities and NaN in x or the weights come out where the index-order float32 sum has them, in every form."""
+    w, x = normal((rows, cols), seed=n + rows), normal((n, cols), seed=cols)
+    x[n // 2, 3], x[n - 1, cols - 1], w[rows - 1, 0], w[rows // 2, cols - 2] = np.inf, np.nan, -np.inf, np.inf
+    x[0, cols - 2] = 0.0  # (times the infinite weight: not a number)
+    y = hip.alloc(n * rows * 4)
+    hip.gemm_dense(S.GpuTensor(F32_TYPE, rows, cols, up(hip, w)), n, up(hip, x), cols, y, rows, S.ACT_STORE)
+    want = np.zeros((n, rows), np.float32)
+    with np.errstate(invalid="ignore"):
+        for k in range(cols):
+            want += x[:, k:k + 1] * w[None, :, k]
+    np.testing.assert_array_equal(hip.get(y, np.float32, n * rows).reshape(n, rows), want)
+
+
+@pytest.mark.parametrize("ty", ggml.TYPES)
+def test_few_positions_non_finite_scales(hip, ty):
+    """Super-blocks whose f16 scales are infinite or not a number: the forms for few positions (GEMM, tile list, several
+    inputs) give what gemm_kernel gives, in the affected rows as in the others."""
+    rows, cols, n = 40, 768, 9
+    w, x = random_blocks(ty, rows, cols, seed=ty), normal((n, cols), seed=3)
+    bb, off = ggml.block_bytes(ty), ggml.F16_FIELDS[ty][0]
+    for r, b, bits in ((3, 1, 0x7C00), (17, 0, 0xFC00), (39, 2, 0x7E00)):
+        w[r, b * bb + off:b * bb + off + 2] = np.frombuffer(np.uint16(bits).tobytes(), np.uint8)
+    t, xb, y = hip.upload_tensor(ty, w), up(hip, x), hip.alloc(n * rows * 4)
+    st = up(hip, np.array([[t.ptr, n << 32]], np.uint64))
+
+    def get():
+        return hip.get(y, np.float32, n * rows).reshape(n, rows)
+
+    hip.gemm(ty, rows, cols, st, 1, xb, cols, n, 0, y, rows, S.ACT_STORE)
+    want = get()
+    assert not np.isfinite(want[:, [3, 17, 39]]).any() and np.isfinite(np.delete(want, [3, 17, 39], axis=1)).all()
+    hip.gemm(ty, rows, cols, st, 1, xb, cols, n, 0, y, rows, S.ACT_STORE | S.SMALL_TILES)
+    np.testing.assert_array_equal(get(), want)
+    hip.gemm_dense(t, n, xb, cols, y, rows, S.ACT_STORE)
+    np.testing.assert_array_equal(get(), want)
+    if ty != ggml.Q8_0:  # (its GEMV adds a row's blocks in another order)
+        hip.gemvn(t, xb, cols, y, rows, 4)
+        np.testing.assert_array_equal(get()[:4], want[:4])
 
 
 # one block up to 4096 pairs, three launches beyond
