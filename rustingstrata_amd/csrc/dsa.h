@@ -43,8 +43,8 @@ template <bool Q5> struct DsaQ45 {
 };
 template <> struct Dsa<Q4_K> : DsaQ45<false> {};
 template <> struct Dsa<Q5_K> : DsaQ45<true> {};
-// (IQ2_XXS keeps the digit planes: its per-group header reads made this form slower, 0.105 -> 0.126 ms for the
-// configs[3] 512-token GEMM)
+// (IQ2_XXS keeps the digit planes: its per-group header reads made this form slower, 0.105 -> 0.126 ms for a
+// 512-token GEMM of 128 experts of 2048 x 768)
 template <> struct Dsa<IQ2_XXS> {
     static constexpr bool ON = false, MIN = false;
     struct Row {};

@@ -28,7 +28,7 @@ struct GemmLaunch {
     // 16-byte aligned)
     bool pair = false;
     int64_t w2 = 0;
-    // tiles of a few dozen positions: the 64-position kernel with two steps of loads in flight (gemm_small.hip)
+    // tiles of a few dozen positions: the 64-position kernel (gemm_small.hip), or the form for few positions
     bool small = false;
 };
 hipError_t launch_gemm(const GemmLaunch& g, hipStream_t s);

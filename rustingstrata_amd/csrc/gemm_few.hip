@@ -9,8 +9,9 @@
 //     side by side and the sum keeps its bits;
 //   * otherwise (rows of few super-blocks, many items) every wave walks its own item's super-blocks with the sum in
 //     registers, and no wave waits for another.
-// (16 positions a unit: 32 or 64, with the weights decoded once for them, spill at two blocks a CU and measure slower,
-// 5120 x 2048 Q6_K: 24 positions 13.4 against 10.1 us, 64 positions 17.8 against 14.7.)
+// (16 positions a unit: 32 or 64, with the weights decoded once for them, measure slower, 5120 x 2048 Q6_K: 24 positions
+// 13.4 against 10.1 us, 64 positions 17.8 against 14.7. At 16 the block form of Q6_K spills 3 registers, the others none; a
+// spill's loads and stores can only make wait_vm<NXL> wait for more than the raw rows, which are older than they are.)
 // X fragments come straight from global memory (the whole X is a few KB to a few hundred: L2), raw weight rows through
 // a wave's own LDS region, reloaded for its next unit as soon as the current one is decoded. Two blocks fit a CU.
 #include <algorithm>
@@ -34,8 +35,9 @@ constexpr int FPP = FPM + 4;  // floats of a term row (16-byte pad: rows start i
 // items): Q6_K 5120 x 2048: 5 positions 28.4 -> 7.2, 24 29.6 -> 9.9, 64 (1280 items) 32.1 -> 15.0, 256 (5120) 32.4 ->
 // 36.7; Q4_K 5120 x 2048: 64 27.8 -> 15.7, 100 (2240) 27.8 -> 23.9, 200 28.4 -> 42.7; 2048 x 2048, 256 positions
 // (2048): Q6_K 31.8 -> 16.2, Q4_K 27.8 -> 20.5. One unit of positions, whatever the rows: 151936 x 2048, 16 positions
-// (9496): Q6_K 128 -> 69, Q4_K 95 -> 92, Q2_K 82 -> 54 (32 positions: 134 -> 128, 103 -> 179, 87 -> 103). A block an item up to 1280 items: 64 positions of 5120 x 2048 15.0
-// against 16.1 a wave an item (Q4_K 15.7 / 20.1), 256 of 2048 x 2048 22.2 / 16.2 (23.2 / 20.5).
+// (9496): Q6_K 128 -> 69, Q4_K 95 -> 92, Q2_K 82 -> 54 (32 positions: 134 -> 128, 103 -> 179, 87 -> 103). A block an item up
+// to 1280 items: 64 positions of 5120 x 2048 15.0 against 16.1 a wave an item (Q4_K 15.7 / 20.1), 256 of 2048 x 2048 22.2 /
+// 16.2 (23.2 / 20.5).
 constexpr long long FEW_DENSE_BLOCK_ITEMS = 1280, FEW_DENSE_ITEMS = 2048;
 long long few_dense_items(int rows, int n) { return (long long)((rows + 15) / 16) * ((n + FPM - 1) / FPM); }
 // Tile lists with SMALL_TILES, gemm_small_kernel -> this form.

@@ -3,7 +3,7 @@
 // kernels gemmi_q / gemms_*, src/cuda/kernels.cu:1355-1497, chosen by tile size in src/cuda/mod.rs:587-620).
 //
 // With few positions a block's super-block step is short (the 16 rows a wave decodes, then one or two MFMA tile
-// pairs), so a weight load issued one step ahead does not land in time. The types whose kernel fits 128 registers
+// pairs), so a weight load issued one step ahead does not land in time. The types that take less time so
 // (small_two) run two blocks a CU, each one step ahead, and wait for all loads at a step's end; the others run one
 // block a CU that keeps two steps in flight:
 //   * a block takes 64 positions x 128 weight rows (8 waves, 16 rows each, as gemm_kernel; pair mode 64 gate + 64 up);
@@ -34,10 +34,12 @@ constexpr int SXI = SM * 16 / 64 / SW;  // X load instructions per wave and step
 constexpr int SDX = SW * SM;            // floats of one scale buffer (a copy per wave)
 }  // namespace
 
-// Two blocks a CU, each one step ahead (X in 2 slots, raw rows in 1), for the types whose kernel fits 128 registers: the
-// other block's waves cover a step's waits better than a second step in flight does. 512-token GEMMs over 128 experts,
-// us with one block / two: Q2_K gate/up 114 / 81, IQ2_XXS 168 / 121, Q3_K down 89 / 70 (1000 tokens 141 / 109, 204 / 148,
-// 115 / 91); the others spill and lose (Q6_K down 84 / 99, IQ4_XS gate/up 128 / 261).
+// Two blocks a CU, each one step ahead (X in 2 slots, raw rows in 1), for the types that measured faster so: the other
+// block's waves cover a step's waits better than a second step in flight does, and these kernels lose little to the 128
+// registers (4, 6 and 1 of them spilled for Q2_K, Q3_K and IQ2_XXS; all waits of this form are for every load, so the
+// spills do not upset a count). 512-token GEMMs over 128 experts, us with one block / two: Q2_K gate/up 114 / 81, IQ2_XXS 168
+// / 121, Q3_K down 89 / 70 (1000 tokens 141 / 109, 204 / 148, 115 / 91); the others need 149 to 205 registers and lose (Q6_K
+// down 84 / 99, IQ4_XS gate/up 128 / 261).
 __host__ __device__ constexpr bool small_two(int T) { return T == Q2_K || T == Q3_K || T == IQ2_XXS; }
 
 template <int T> struct SmallFmt : GemmPlanes<T> {
