@@ -423,9 +423,10 @@ class HipBackend:
                                      strides, int(tiles), max_tiles, int(n_tiles_dev), int(err_dev), chunk))
 
     # Routed rows per expert (T k / E) up to which a prefill MoE block takes 64-position tiles and the
-    # 64-position GEMM kernel (SMALL_TILES); above it, tiles of gemm_block_positions() (configs[2] layer: 512 tokens,
-    # 32 rows an expert: 0.277 against 0.300 ms; 1024 tokens, 64 rows: 0.358 against 0.373 ms; 2048 tokens, 128
-    # rows: 0.592 against 0.540 ms).
+    # 64-position GEMM kernel (SMALL_TILES); above it, tiles of gemm_block_positions(). Time of the former over that of the
+    # latter at 48 / 64 / 96 / 128 rows an expert (2048 x 768, 128 experts top 8, even load): Q6_K 0.81 / 0.99 / 1.24 / 1.35,
+    # Q4_K 0.79 / 0.95 / 1.16 / 1.28, Q2_K 0.57 / 0.73 / 0.88 / 0.96; with a Zipf-skewed load 0.80 / 0.82 / 0.91 / 0.96, 0.77
+    # / 0.82 / 0.94 / 1.03, 0.60 / 0.63 / 0.72 / 0.79.
     SMALL_TILE_ROWS = 64
 
     def moe_tile_plan(self, t, k, n_expert, small=None):

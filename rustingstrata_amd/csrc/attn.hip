@@ -565,7 +565,7 @@ hipError_t launch_attn_decode(const float* q, const uint16_t* kc, const uint16_t
 //   of sub-tile mt make the 8 K-elements of a k-step, and V^T's A fragment reads the same keys).
 // A wave issues 64 MFMAs of 32 cycles a key tile (2048 cycles: with the hi / lo splits 275 GFLOP for 4096 tokens, 32
 // heads of 128 over 4) and ~270 other VALU instructions, 32 of them quarter-rate exps: the two overlap between the two
-// waves of a SIMD for 54% MFMA time. Measured there 273 us; 381 with 16 x 16 MFMAs (a SIMD issues about two VALU
+// waves of a SIMD for 54% MFMA time. Measured there 276-283 us; 381 with 16 x 16 MFMAs (a SIMD issues about two VALU
 // instructions beside an MFMA of 16 cycles, so half the MFMAs leave room for more), a rescale of the accumulators in most
 // tiles, the weights' scale and f16 remainders as instructions of their own and four cross-lane steps a tile. Rows of one
 // tile instead of two from opposite ends keep a sliding window's key range short (window 1024: 545 -> 147 us).

@@ -513,7 +513,7 @@ static hipError_t gemm_t(const GemmLaunch& g, hipStream_t s) {
 // SIMD, 62 us at 2.1 GHz, against 16 us of MFMAs), so it is built to keep three blocks a CU (three waves a SIMD that
 // share no barrier) at work: a block of 4 waves takes 64 rows x 64 positions, wave w rows 16 w .. 16 w + 15; X rows come
 // by direct global-to-LDS loads one 256-value step ahead (two buffers), raw weight rows into the wave's own LDS region
-// as soon as its current ones are decoded. 4096 x 2048 x 2048: 85 us (172 with 64 x 128 blocks whose loads went
+// as soon as its current ones are decoded. 4096 x 2048 x 2048: 80-91 us (172 with 64 x 128 blocks whose loads went
 // through registers, two barriers a step and two half-empty K=64 MFMAs a pair of blocks).
 constexpr int Q8_ROWS = 64, Q8_POS = 64, Q8_SB = 272, Q8_NT = Q8_POS / 16;
 constexpr int Q8_NCH = 19;            // 16-byte chunks of a raw row's LDS pitch: 18 cover 272 bytes at any 2-byte offset, odd
