@@ -1,14 +1,14 @@
-"""Benchmark of the quantized-matmul hot path on one MI355X (BASELINE.json: "Q-GEMV achieved HBM GB/s (% peak); MoE
+"""Benchmark of the quantized-matmul hot path on one MI355X ("Q-GEMV achieved HBM GB/s (% peak); MoE
 grouped-GEMM prefill tok/s at 4K").
 
-Workload (`value`): BASELINE.json configs[1], the batch-1 decode GEMV sweep: Q4_K, Q5_K, Q6_K and Q8_0 at 6144x2048
+Workload (`value`): the batch-1 decode GEMV sweep: Q4_K, Q5_K, Q6_K and Q8_0 at 6144x2048
 (fused QKV), 2048x2048 and 151936x2048 (lm head); weights seeded N(0, 0.02) quantized by the library's quantizer,
 x seeded N(0, 1). A step is one pass over the 12 GEMVs; value = algorithmic bytes (weights + x + y) of the timed
 steps / their time (GB/s). Each GEMV rotates over distinct weight copies totalling > 512 MB, so the 256 MB
 Infinity Cache cannot serve repeats (the reference harness reads one copy, tests/kernels.rs:270-331).
 
 Also reported: per-shape GB/s, the roofline of the dominant kernel (the Q4_K lm-head GEMV, the reference's own
-headline shape), the Qwen3-30B-A3B-shaped MoE layer (configs[2]) at 4096 tokens (tok/s and int8 MFMA fraction of
+headline shape), the Qwen3-30B-A3B-shaped MoE layer at 4096 tokens (tok/s and int8 MFMA fraction of
 its grouped GEMMs) and at 1 token (decode GB/s), and the reference's CPU path (the oracle's C restatement of
 cpu_moe::matvec) timed on this host on a bounded sample.
 
@@ -194,7 +194,7 @@ def gemm_digit_planes(ggml, ty):
 
 
 def bench_moe(hip, S, ggml, T, iters, ty_gu=None, ty_d=None, small=None):
-    """E=128, top-8, H=2048, I=768; gate/up Q5_K, down Q6_K (or the given types, e.g. configs[4]'s
+    """The MoE layer: E=128, top-8, H=2048, I=768; gate/up Q5_K, down Q6_K (or the given types, e.g. the 48-layer stack's
     Q2_K / Q3_K experts); Zipf-skewed routing; T tokens. small: the 64-position GEMM kernel over 64-position tiles
     (None: the backend's choice for T k / E routed rows per expert)."""
     E, H, F, k = 128, 2048, 768, 8
@@ -254,7 +254,7 @@ def bench_moe(hip, S, ggml, T, iters, ty_gu=None, ty_d=None, small=None):
     # per kernel: the gate/up launch (its x quantization included) and the down launch (h quantization included);
     # issued int8 ops count every digit plane (the MFMA work done), useful ops the matrix product
     # HBM bytes per launch of each GEMM from rocprofv3 FETCH_SIZE / WRITE_SIZE scaled by a copy kernel
-    # (profiles/moe_prefill_4k.md, the 4096-token configs[2] layer); None for other shapes or when absent
+    # (profiles/moe_prefill_4k.md, the 4096-token MoE layer); None for other shapes or when absent
     traffic = {}
     prof = os.path.join(ROOT, "profiles", "moe_prefill_4k.md")
     if T == 4096 and ty_gu == ggml.Q5_K and ty_d == ggml.Q6_K and os.path.exists(prof):
@@ -284,7 +284,7 @@ def bench_moe(hip, S, ggml, T, iters, ty_gu=None, ty_d=None, small=None):
 
 
 def bench_moe_decode(hip, S, ggml, iters):
-    """configs[2] at 1 token: route + paired gate/up moe_gemv as one launch (h quantized inside it) -> swiglu_q +
+    """The MoE layer at 1 token: route + paired gate/up moe_gemv as one launch (h quantized inside it) -> swiglu_q +
     moe_down_combine as one down GEMV (the SwiGLU quantized inside it) + combine (src/gpu_model.rs:3383-3412), over 2 copies of the 128 experts
     (884 MB, past the Infinity Cache)."""
     E, H, F, k = 128, 2048, 768, 8
@@ -361,7 +361,7 @@ def bench_moe_decode(hip, S, ggml, iters):
 
 
 def bench_attn_decode(hip, S, positions=(255, 1023, 4099), layers=48):
-    """configs[4]'s decode attention alone (32 query heads over 4 KV heads of 128, f16 caches): attn_decode + its
+    """The 48-layer stack's decode attention alone (32 query heads over 4 KV heads of 128, f16 caches): attn_decode + its
     split merge over `layers` caches in turn (past the Infinity Cache at 4K), replayed from a recorded graph; the
     K/V bytes a call reads and the time per call at each position."""
     nh, nkv, hd = 32, 4, 128
@@ -405,7 +405,7 @@ def bench_attn_decode(hip, S, positions=(255, 1023, 4099), layers=48):
 
 
 def codebook_blocks(ggml, ty, rows, cols, seed):
-    """configs[3] weights: grid indices, sign bits and sub-block scales uniform from a seed (random block bytes), with
+    """Codebook expert weights: grid indices, sign bits and sub-block scales uniform from a seed (random block bytes), with
     each block's f16 d set to 2^-6 so every value is finite."""
     rng = np.random.default_rng(seed)
     bb = ggml.block_bytes(ty)
@@ -443,7 +443,7 @@ def bench_dense_gemm(hip, S, ggml, iters=20):
 
 
 def bench_codebook(hip, S, ggml, iters):
-    """configs[3]: IQ2_XXS / IQ3_S / IQ4_XS experts of 2048 x 768 (out x in), 128 experts.
+    """IQ2_XXS / IQ3_S / IQ4_XS experts of 2048 x 768 (out x in), 128 experts.
     T = 1: moe_gemv over 8 Zipf-routed experts, the 128 experts rotated over copies past 512 MB (GB/s of the 8 experts'
     bytes). T = 512: route -> device sort -> grouped GEMM over the 128 experts (int8 TOP/s on routed pairs)."""
     E, rows, cols, k = 128, 2048, 768, 8
@@ -509,7 +509,7 @@ def bench_codebook(hip, S, ggml, iters):
 
 
 def bench_stack(hip, S, ggml, n_prompt=4096, n_decode=128, chunk=4096, n_layer=48):
-    """the 48-layer Qwen3-30B-A3B-shaped stack, random-init on the device (Q2_K gate/up and Q3_K down
+    """The 48-layer Qwen3-30B-A3B-shaped stack, random-init on the device (Q2_K gate/up and Q3_K down
     experts, Q6_K attention, Q8_0 embeddings and output head), every expert resident. A uniform-random prompt of 4096
     token ids is prefilled in chunks of `chunk` (4096: the reference's prefill chunk when it is not calibrated,
     src/main.rs:30,407), then 128 greedy tokens are decoded (each a recorded-graph replay after the first; the host
@@ -572,7 +572,7 @@ def cpu_info():
 def cpu_baseline(shapes, budget_s=10.0):
     """The reference CPU path restated in C (oracle/): cpu_moe::matvec over the same GEMV sweep with the AVX2 dots the
     reference dispatches to on x86-64-v3 (src/cpu_moe.rs:1364-1391), threads over 32-row chunks like rayon's
-    par_chunks_mut(32); beside it the scalar dots, one thread, and the configs[0] GEMV and configs[2] MoE layer."""
+    par_chunks_mut(32); beside it the scalar dots, one thread, and the 4096 x 4096 GEMV and the MoE layer."""
     from oracle import oracle as O
     info = cpu_info()
     threads = info["threads"]
@@ -599,7 +599,7 @@ def cpu_baseline(shapes, budget_s=10.0):
                          "(C restatement of cpu_moe::matvec and its x86-64-v3 kernels)"}
         small = [s for s in shapes if s["rows"] == 6144]
         out["one_thread_GB/s"] = round(sweep_rate(2.0, 1, small)[0], 2)
-        # configs[0]: Q4_K 4096 x 4096
+        # Q4_K 4096 x 4096
         import rustingstrata_amd as S
         from rustingstrata_amd import ggml
         w0 = synth_weights(S, ggml, ggml.Q4_K, 4096, 4096, seed=999)
@@ -611,7 +611,7 @@ def cpu_baseline(shapes, budget_s=10.0):
         us0 = 1e6 * (time.time() - t0) / n0
         out["config0_q4k_4096x4096"] = {"us": round(us0, 1), "GB/s": round((w0.nbytes + 32768) / us0 / 1e3, 2),
                                         "threads": threads}
-        # configs[2] on the CPU: cpu_moe::experts_multi over 64 tokens of the MoE layer (E=128, top-8, Q5_K gate/up,
+        # the MoE layer on the CPU: cpu_moe::experts_multi over 64 tokens of the MoE layer (E=128, top-8, Q5_K gate/up,
         # Q6_K down; 16 distinct experts repeated)
         E, H, F, k, T = 128, 2048, 768, 8, 64
         rng = np.random.default_rng(13)
@@ -628,7 +628,7 @@ def cpu_baseline(shapes, budget_s=10.0):
         dt = time.time() - t0
         out["moe_layer"] = {"tok_per_s": round(T / dt, 1), "ms_per_token": round(1000 * dt / T, 3), "tokens": T,
                             "cores": threads, "variant": "avx2",
-                            "sample": "cpu_moe::experts_multi restated in C, 64 tokens of configs[2] (routing: N(0,1) "
+                            "sample": "cpu_moe::experts_multi restated in C, 64 tokens of the MoE layer (routing: N(0,1) "
                                       "logits + 8 * rank^-1.1 over a seeded expert permutation, seed 13)"}
     finally:
         O.set_avx2(False)
@@ -682,16 +682,16 @@ def main():
     ap.add_argument("--profile-gemv", action="store_true",
                     help="only run the Q4_K lm-head GEMV and a 256 MB copy kernel 50 times each (for rocprofv3)")
     ap.add_argument("--profile-moe", action="store_true",
-                    help="only run the configs[2] MoE prefill layer at 4096 and 512 tokens (--moe-iters times each) "
+                    help="only run the MoE prefill layer at 4096 and 512 tokens (--moe-iters times each) "
                          "and a 256 MiB copy kernel as often (for rocprofv3)")
     ap.add_argument("--profile-attn", action="store_true",
-                    help="only configs[4]'s decode attention (+ merge) at 256, 1024 and 4100 positions")
+                    help="only the stack's decode attention (+ merge) at 256, 1024 and 4100 positions")
     ap.add_argument("--profile-decode", action="store_true",
-                    help="only run the configs[2] 1-token MoE decode layer 200 times, eagerly (for rocprofv3)")
+                    help="only run the 1-token MoE decode layer 200 times, eagerly (for rocprofv3)")
     ap.add_argument("--eager", action="store_true", help="launch every op from the host (no recorded graphs)")
-    ap.add_argument("--no-stack", action="store_true", help="skip the configs[4] 48-layer stack")
+    ap.add_argument("--no-stack", action="store_true", help="skip the 48-layer stack")
     ap.add_argument("--floor-only", action="store_true", help="only the GEMV sweep and its launch / read floors")
-    ap.add_argument("--stack-only", action="store_true", help="only run the configs[4] 48-layer stack")
+    ap.add_argument("--stack-only", action="store_true", help="only run the 48-layer stack")
     args = ap.parse_args()
     global USE_GRAPHS
     USE_GRAPHS = not args.eager
@@ -736,7 +736,7 @@ def main():
     roof = roofline_q4k_lmhead(hip, shapes, xb, yb)
     log(f"[bench] Q4_K lm head: {roof['achieved']} GB/s ({100 * roof['frac']:.1f}% of peak)")
     extra = {}
-    # configs[0] on the GPU: Q4_K 4096 x 4096 (9.47 MB), rotated copies, graph replays
+    # on the GPU: Q4_K 4096 x 4096 (9.47 MB), rotated copies, graph replays
     b1 = synth_weights(S, ggml, ggml.Q4_K, 4096, 4096, seed=999)
     r1 = Rotated(hip, S, ggml.Q4_K, b1, 4096, 4096)
     x1, y1 = hip.upload(np.random.default_rng(8).standard_normal(4096).astype(np.float32)), hip.alloc(4096 * 4)
@@ -745,8 +745,8 @@ def main():
     extra["config0_q4k_4096x4096"] = {"us": round(us1, 2), "GB/s": round(by1 / us1 / 1e3, 1),
                                       "pct_peak": round(100 * by1 / us1 / 1e3 / HBM_PEAK_GBS, 1)}
     hip.drop_graphs()
-    log(f"[bench] configs[0] Q4_K 4096x4096: {extra['config0_q4k_4096x4096']}")
-    # configs[4]'s expert types as decode GEMVs (the Q8_0 lm head is in the sweep)
+    log(f"[bench] Q4_K 4096x4096: {extra['config0_q4k_4096x4096']}")
+    # the 48-layer stack's expert types as decode GEMVs (the Q8_0 lm head is in the sweep)
     ud = {}
     for name, rows, cols in (("Q2_K", 6144, 2048), ("Q2_K", 2048, 2048), ("Q3_K", 6144, 2048), ("Q3_K", 2048, 2048),
                              ("Q2_K", 151936, 2048), ("Q3_K", 151936, 2048)):
@@ -760,7 +760,7 @@ def main():
         hip.drop_graphs()
         del rr
     extra["gemv_config4_types"] = ud
-    log(f"[bench] configs[4] types GEMV: {ud}")
+    log(f"[bench] stack types GEMV: {ud}")
     extra["floor"] = bench_floor(hip, shapes, per_shape)
     log(f"[bench] launch / read floors: {extra['floor']}")
     if not args.no_moe:
@@ -774,10 +774,10 @@ def main():
         extra["codebook_experts"] = bench_codebook(hip, S, ggml, 100)
         extra["gemm_dense_4k"] = bench_dense_gemm(hip, S, ggml)
         log(f"[bench] dense GEMMs 4096 x 2048 x 2048: {extra['gemm_dense_4k']}")
-        log(f"[bench] configs[3] codebook experts: {extra['codebook_experts']}")
+        log(f"[bench] codebook experts: {extra['codebook_experts']}")
     if not args.no_stack:
         extra["stack_config4"] = bench_stack(hip, S, ggml)
-        log(f"[bench] configs[4] 48-layer stack: {extra['stack_config4']}")
+        log(f"[bench] 48-layer stack: {extra['stack_config4']}")
     cpu = None if args.no_cpu else cpu_baseline(shapes)
     out = {
         "metric": "Q-GEMV achieved HBM GB/s (% peak); MoE grouped-GEMM prefill tok/s at 4K",

@@ -75,7 +75,7 @@ def test_size_helpers():
 
 
 def test_config4_shape():
-    """the Qwen3-30B-A3B-shaped stack (48 layers, hidden 2048, 32 query heads over 4 KV heads of 128,
+    """The Qwen3-30B-A3B-shaped stack (48 layers, hidden 2048, 32 query heads over 4 KV heads of 128,
     128 experts top-8 of intermediate 768, vocabulary 151936) with the UD-Q2_K_XL-like mix (Q2_K/Q3_K experts, Q6_K
     attention, Q8_0 embeddings and output)."""
     from rustingstrata_amd.qwen3moe import Config

@@ -28,10 +28,15 @@ def test_f32_gemm_form(n, rows, form):
 
 
 def test_f32_gemm_form_of_any_size():
+    """A form for every size, and its blocks of rows within what HIP takes along y up to the rows that one form of 16 rows a
+    block took."""
     f = rule("_ZN6strata13gemm_f32_formEiii", ctypes.c_int, ctypes.c_int, ctypes.c_int)
     for n in (1, 2, 63, 64, 65, 4097, 1 << 20, 1 << 30):
         for rows in (1, 3, 16, 17, 151936, 1 << 20, 1 << 30):
             assert f(n, rows, CUS) in (0, 1, 2, 4)
+    for n in (1, 2, 3, 8, 17, 33, 64, 65, 128, 129, 1000, 4096):
+        for rows in (262140, 262141, 524280, 524281, 1000003, 16 * 65535):
+            assert -(-rows // (4 * (f(n, rows, CUS) or 4))) <= 65535
 
 
 @pytest.mark.parametrize("ty,nt,cols,tiles,pads", [

@@ -1,7 +1,7 @@
-"""BASELINE configs at their stated workloads on the GPU, through the C ABI, against the CPU oracle.
+"""The benchmarked workloads on the GPU, through the C ABI, against the CPU oracle.
 
-one Q4_K 4096 x 4096 dequant-GEMV, weights from the repo quantizer over seeded N(0, 0.02).
-configs[3]: IQ2_XXS / IQ3_S / IQ4_XS experts (128 of them, 2048 x 768 each, random grid indices, signs and scales),
+One Q4_K 4096 x 4096 dequant-GEMV, weights from the repo quantizer over seeded N(0, 0.02).
+IQ2_XXS / IQ3_S / IQ4_XS experts (128 of them, 2048 x 768 each, random grid indices, signs and scales),
 T = 1 through moe_gemv over the 8 routed slots and T = 512 through route -> moe_sort -> gemm_grouped.
 Bars as in test_gpu_parity: fp32 within max relative error 1e-3; the CPU dot's bits where the close is exact.
 """

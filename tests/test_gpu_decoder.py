@@ -260,7 +260,7 @@ def test_attn_prefill_sink_gate_window(hip):
 
 
 def test_attn_prefill_full_size(hip):
-    """configs[4]'s layer shape at its full prompt: 4096 tokens, 32 query heads over 4 KV heads of 128; rows sampled
+    """The 48-layer stack's layer shape at its full prompt: 4096 tokens, 32 query heads over 4 KV heads of 128; rows sampled
     over the whole triangle (every 64th, plus the last)."""
     rows = list(range(0, 4096, 64)) + [4095]
     prefill_case(hip, 32, 4, 128, 4096, 0, seed=30, rows=rows)

@@ -142,7 +142,7 @@ def mid_rows(hip, m, c, n):
 
 CFGS = {
     "small": small_cfg,
-    # the configs[4] head shape: head_dim 128, 8 query heads over each KV head
+    # the 48-layer stack's head shape: head_dim 128, 8 query heads over each KV head
     "hd128_gqa8": lambda: Config(n_layer=2, n_embd=1024, n_head=16, n_head_kv=2, head_dim=128, n_expert=16,
                                  n_expert_used=4, n_ff_exp=256, n_vocab=300),
     # a hidden size past the fused FFN-norm + router launch (its unfused form)
@@ -262,7 +262,7 @@ def test_models_in_sequence_keep_their_own_graphs(hip):
 
 
 def test_config4_full_workload(hip):
-    """configs[4] at its workload: the 48-layer Qwen3-30B-A3B-shaped random model, a 4096-token uniform-random prompt
+    """The 48-layer Qwen3-30B-A3B-shaped random model, a 4096-token uniform-random prompt
     prefilled, then 128 greedy decode tokens.
 
     * The prompt in one chunk of 4096 and in two of 2048 gives the same logits and KV caches, bit for bit (per-token

@@ -299,7 +299,7 @@ def test_gemv_matches_cpu_matvec(hip, ty, rows, cols):
 @pytest.mark.parametrize("ty", [ggml.Q4_K, ggml.Q5_K, ggml.Q6_K, ggml.Q8_0])
 @pytest.mark.parametrize("rows", [6144, 151936])
 def test_gemv_sweep_shapes(hip, ty, rows):
-    """configs[1] at full size (the fused-QKV-like and lm-head-like shapes, 2048 columns): every row against the
+    """The decode GEMV sweep at full size (the fused-QKV-like and lm-head-like shapes, 2048 columns): every row against the
     oracle's cpu_moe::matvec (tiles of many rows: a row past a tile's loaded bytes would show here)."""
     cols = 2048
     w = random_blocks(ty, rows, cols, seed=rows + ty)
@@ -919,7 +919,7 @@ def test_moe_prefill_layer_matches_experts_multi(hip):
 
 
 def test_moe_prefill_layer_full_size(hip):
-    """configs[2] at its full size (128 experts, hidden 2048, intermediate 768, top-8, 4096 tokens, Zipf-skewed
+    """The MoE layer at its full size (128 experts, hidden 2048, intermediate 768, top-8, 4096 tokens, Zipf-skewed
     routing): the device layer against cpu_moe::experts_multi on every token, and the fused gate/up launch equal to
     the two-call sequence bit for bit."""
     E, H, F, T, k = 128, 2048, 768, 4096, 8
@@ -935,7 +935,7 @@ def test_moe_prefill_layer_full_size(hip):
 
 
 def test_moe_prefill_layer_512_tokens(hip):
-    """configs[2] at its 512-token size (128 experts, Zipf-skewed: most experts get a few dozen routed rows, so the
+    """The MoE layer at its 512-token size (128 experts, Zipf-skewed: most experts get a few dozen routed rows, so the
     grouped GEMMs run their small-tile form): the device layer against cpu_moe::experts_multi on every token, fused
     and unfused gate/up bit for bit."""
     E, H, F, T, k = 128, 2048, 768, 512, 8
@@ -982,7 +982,7 @@ def run_prefill(hip, E, H, F, T, k, gate, upw, dn, hs, logits, fused=False, smal
 
 def test_moe_decode_layer_matches_experts(hip):
     """The decode sequence of src/gpu_model.rs:3383-3412: moe_route -> paired gate/up moe_gemv -> swiglu_q ->
-    moe_down_combine, against cpu_moe::experts, at configs[2]'s shape (128 experts)."""
+    moe_down_combine, against cpu_moe::experts, at the MoE layer's shape (128 experts)."""
     E, H, F, k = 128, 2048, 768, 8
     gate, upw, dn = moe_weights(E, H, F, seed=50)
     h = normal(H, seed=51)

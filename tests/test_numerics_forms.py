@@ -1,6 +1,6 @@
 """Why the grouped GEMM keeps exact integer digit planes: cheaper MFMA forms miss the 1e-3 parity bound.
 
-The north star's bound for fp32 outputs is a max relative error of 1e-3 (tests/helpers.py max_rel_err: element-wise,
+The bound for fp32 outputs is a max relative error of 1e-3 (tests/helpers.py max_rel_err: element-wise,
 with a floor of 1e-3 of the largest output). These CPU checks take K-quant rows (random blocks, the reference's
 random_tensor design), Q8_K activations (cpu_moe::quantize_q8k), and the exact product of the dequantized values
 (what src/cpu_moe.rs computes, up to f32 rounding). They then apply the number formats a faster GEMM would feed the
