@@ -63,6 +63,8 @@ hipError_t launch_gemv_f32(const float* w, int rows, int cols, const float* x, u
 // gemm_dense with f32 weights: y[m * y_stride + r] (op) W[r] . x[m * x_stride], m < n; act 0 store, 1 SwiGLU, 2 add.
 hipError_t launch_gemm_f32(const float* w, int rows, int cols, const float* x, uint64_t x_stride, float* y,
                            uint64_t y_stride, int n, int act, hipStream_t s);
+// Whether launch_norm_rope's many-heads form stages the value rows of that many heads with ncu CUs.
+bool nr_staged(int heads, int ncu);
 // The form that launch_gemm_f32 takes with ncu CUs: 0 quad, else the rows a wave of the ring form.
 int gemm_f32_form(int n, int rows, int ncu);
 hipError_t launch_fill_blocks(int ty, uint8_t* w, uint64_t n_blocks, uint64_t seed, float lo, float hi, hipStream_t s);

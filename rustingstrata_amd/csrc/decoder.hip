@@ -19,6 +19,15 @@ __device__ __forceinline__ uint16_t f32_to_f16_bits(float v) {
 }
 
 
+// CUs of the device (256 where that cannot be told).
+static int cu_count() {
+    static const int ncu = [] {
+        int dev = 0, v = 0;
+        return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
+    }();
+    return ncu;
+}
+
 // ---- rms_norm + rope (+ KV store) ----
 // One wave per head, n <= 512, the head staged in LDS. The sum of squares runs in index order on one lane (n adds per
 // head, a small part of the launch), and out = x * (1 / sqrt(ss / n + eps)) * w in the reference's operation order,
@@ -139,25 +148,27 @@ __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_kernel(NormRope a) {
 // in LDS with every load issued at once; wave 0 then sums the squares a lane
 // per head (the heads' sequential chains run side by side); each wave then takes 16 consecutive heads, a lane per
 // rope pair (i, i + 64), recomputing the pair's angle only when the position changes. The arithmetic is
-// norm_rope_kernel's, so both kernels give the same bits.
-// (The value rows are read where they are stored, not staged: 33 KB of LDS a block, four a CU instead of two; 1501 tokens x
-// 36 heads 31.3 -> 28.6 us.)
+// norm_rope_kernel's, so both kernels give the same bits. STAGED: the value rows of stored key heads are requested with
+// the heads and wait in LDS (66 KB a block, two a CU), else they are read where they are stored (33 KB, four a CU).
 constexpr int NR_MANY = 64, NR_P = 129;  // heads a block; LDS pitch of a staged head (bank spread for the sums)
+template <bool STAGED>
 __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_many_kernel(NormRope a) {
-    __shared__ float xs[NR_MANY][NR_P];
+    __shared__ float xs[NR_MANY][NR_P], vs[STAGED ? NR_MANY : 1][NR_P];
     __shared__ float ssq[NR_MANY];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int total = a.qrows + a.rows, g0 = (int)blockIdx.x * NR_MANY;
     const float qw0 = a.qrows ? a.qw[lane] : 0.0f, qw1 = a.qrows ? a.qw[lane + 64] : 0.0f;
     const float kw0 = a.rows ? a.w[lane] : 0.0f, kw1 = a.rows ? a.w[lane + 64] : 0.0f;
     // 16-byte chunk c = tid + 256 u of the block: head c / 32, values 4 (c % 32) ..
-    float4 xv[8];
+    float4 xv[8], vv[STAGED ? 8 : 1];
 #pragma unroll
     for (int u = 0; u < 8; u++) {
         const int c = tid + 256 * u, j = c >> 5, g = g0 + j;
         if (g < total) {
             const NrHead h = nr_head(a, g);
             xv[u] = *(const float4*)(h.xr + 4 * (c & 31));
+            if constexpr (STAGED)
+                if (h.vr) vv[u] = *(const float4*)(h.vr + 4 * (c & 31));
         }
     }
 #pragma unroll
@@ -165,6 +176,10 @@ __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_many_kernel(NormRope 
         const int c = tid + 256 * u, j = c >> 5, g = g0 + j, i = 4 * (c & 31);
         if (g < total) {
             xs[j][i] = xv[u].x; xs[j][i + 1] = xv[u].y; xs[j][i + 2] = xv[u].z; xs[j][i + 3] = xv[u].w;
+            if constexpr (STAGED)
+                if (g >= a.qrows && a.kc) {
+                    vs[j][i] = vv[u].x; vs[j][i + 1] = vv[u].y; vs[j][i + 2] = vv[u].z; vs[j][i + 3] = vv[u].w;
+                }
         }
     }
     __syncthreads();
@@ -205,8 +220,9 @@ __global__ __launch_bounds__(64 * NR_WAVES) void norm_rope_many_kernel(NormRope 
             const uint64_t e = ((uint64_t)pos * h.per + h.b % h.per) * 128;
             a.kc[e + lane] = f32_to_f16_bits(o0);
             a.kc[e + lane + 64] = f32_to_f16_bits(o1);
-            a.vc[e + lane] = f32_to_f16_bits(h.vr[lane]);
-            a.vc[e + lane + 64] = f32_to_f16_bits(h.vr[lane + 64]);
+            const float* vr = STAGED ? vs[j] : h.vr;
+            a.vc[e + lane] = f32_to_f16_bits(vr[lane]);
+            a.vc[e + lane + 64] = f32_to_f16_bits(vr[lane + 64]);
         }
     }
 }
@@ -230,6 +246,11 @@ __global__ __launch_bounds__(64 * NR_WAVES) void rope_pairs_kernel(float* x, uin
     }
 }
 
+// Whether the many-heads form stages the value rows: while its blocks all fit at two a CU, where a launch is one block's chain
+// and the rows' latency part of it (128 tokens x 40 heads 13.6 us, 14.8 not staged; 1000 x 32 18.2, 20.9); with more blocks
+// four a CU are faster (1501 x 36 29.0 staged, 26.5 not, 4096 x 36 59.2, 44.4; 1501 x 32 28.0, 23.9).
+bool nr_staged(int heads, int ncu) { return (heads + NR_MANY - 1) / NR_MANY <= 2 * ncu; }
+
 hipError_t launch_norm_rope(const NormRope& a0, hipStream_t s) {
     const int total = a0.qrows + a0.rows;
     if (total <= 0) return hipSuccess;
@@ -243,9 +264,11 @@ hipError_t launch_norm_rope(const NormRope& a0, hipStream_t s) {
     for (int i = 0; i < a.nfreq; i++) a.freq[i] = std::pow((double)a.base, -2.0 * (double)i / (double)a.n_rot);
     const bool vec = ((uintptr_t)a.qx | (uintptr_t)a.x | (uintptr_t)a.v) % 16 == 0 && a.q_stride % 4 == 0 &&
                      a.x_stride % 4 == 0 && a.q_tstride % 4 == 0 && a.x_tstride % 4 == 0 && a.v_tstride % 4 == 0;
-    if (total >= 4 * NR_MANY && vec && a.n == 128 && a.n_rot == 128)  // the many-heads form: 16-byte chunks, heads of 128
-        norm_rope_many_kernel<<<dim3((unsigned)((total + NR_MANY - 1) / NR_MANY)), dim3(64 * NR_WAVES), 0, s>>>(a);
-    else
+    const unsigned many = (unsigned)((total + NR_MANY - 1) / NR_MANY);
+    if (total >= 4 * NR_MANY && vec && a.n == 128 && a.n_rot == 128) {  // the many-heads form: 16-byte chunks, heads of 128
+        if (!nr_staged(total, cu_count())) norm_rope_many_kernel<false><<<dim3(many), dim3(64 * NR_WAVES), 0, s>>>(a);
+        else norm_rope_many_kernel<true><<<dim3(many), dim3(64 * NR_WAVES), 0, s>>>(a);
+    } else
         norm_rope_kernel<<<dim3((unsigned)((total + NR_WAVES - 1) / NR_WAVES)), dim3(64 * NR_WAVES), 0, s>>>(a);
     return hipGetLastError();
 }
@@ -697,12 +720,8 @@ int gemm_f32_form(int n, int rows, int ncu) {
 hipError_t launch_gemm_f32(const float* w, int rows, int cols, const float* x, uint64_t x_stride, float* y,
                            uint64_t y_stride, int n, int act, hipStream_t s) {
     if (!rows || !n) return hipSuccess;
-    static const int ncu = [] {
-        int dev = 0, v = 0;
-        return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
-    }();
     // (the ring's loads into LDS take 16-byte aligned weight rows, the quad form any float's address)
-    switch ((uintptr_t)w % 16 ? 0 : gemm_f32_form(n, rows, ncu)) {
+    switch ((uintptr_t)w % 16 ? 0 : gemm_f32_form(n, rows, cu_count())) {
     case 0: {
         constexpr int P = 2, U = 8;
         const dim3 grid((unsigned)((n + 4 * P - 1) / (4 * P)), (unsigned)((rows + 15) / 16));

@@ -109,3 +109,10 @@ def test_q8_0_grid(total):
     g = f(total)
     assert g.x % 8 == 0 and g.x * 256 < 1 << 32 and 0 < g.y < 1 << 16 and g.z == 1
     assert g.x * g.y >= total
+
+
+@pytest.mark.parametrize("heads,staged", [(256, 1), (128 * 40, 1), (64 * 512, 1), (64 * 512 + 1, 0), (1501 * 36, 0)])
+def test_norm_rope_staged_values(heads, staged):
+    f = rule("_ZN6strata9nr_stagedEii", ctypes.c_int, ctypes.c_int)
+    f.restype = ctypes.c_bool
+    assert f(heads, CUS) == bool(staged)

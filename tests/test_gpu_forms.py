@@ -306,6 +306,37 @@ def test_few_positions_non_finite_scales(hip, ty):
         np.testing.assert_array_equal(get()[:4], want[:4])
 
 
+# 64 heads a block: 512 blocks stage the value rows, more read them where they are stored
+@pytest.mark.parametrize("t", [910, 911, 1501])
+def test_norm_rope_many_heads_in_chunks(hip, t):
+    """A prefill chunk's normed and rotated heads and its KV rows have the bits that the same tokens get as a chunk of 600 (value
+    rows staged), one of 5 (a wave a head) and the rest; the value rows are the f16 roundings."""
+    nh, nkv, hd, pos = 32, 4, 128, 7
+    w = (nh + 2 * nkv) * hd
+    qkv = normal((t, w), seed=t)
+    qw, kw = normal((hd,), seed=1), normal((hd,), seed=2)
+    xb, qwb, kwb = up(hip, qkv), up(hip, qw), up(hip, kw)
+    n = pos + t
+
+    def run(chunks):
+        q, k, kc, vc = (hip.alloc(b) for b in (t * nh * hd * 4, t * nkv * hd * 4, n * nkv * hd * 2, n * nkv * hd * 2))
+        hip.memset(kc), hip.memset(vc)
+        i = 0
+        for c in chunks:
+            x = int(xb) + 4 * w * i
+            hip.rms_norm_rope_qk_t(x, w, hd, qwb, int(q) + 4 * nh * hd * i, c * nh, nh, x + 4 * nh * hd, w, kwb,
+                                   int(k) + 4 * nkv * hd * i, c * nkv, nkv, hd, 1e-6, hd, up(hip, np.array([pos + i, 0], np.int32)),
+                                   1e6, x + 4 * (nh + nkv) * hd, w, kc, vc)
+            i += c
+        return (hip.get(q, np.uint32, t * nh * hd), hip.get(k, np.uint32, t * nkv * hd), hip.get(kc, np.uint16, n * nkv * hd),
+                hip.get(vc, np.uint16, n * nkv * hd))
+
+    one = run([t])
+    assert all(np.array_equal(a, b) for a, b in zip(one, run([600, 5, t - 605])))
+    v = qkv[:, (nh + nkv) * hd:].astype(np.float16).view(np.uint16).reshape(-1)
+    assert np.array_equal(one[3], np.concatenate([np.zeros(pos * nkv * hd, np.uint16), v]))
+
+
 # one block up to 4096 pairs, three launches beyond
 @pytest.mark.parametrize("t,k,E,chunk", [(1, 1, 1, 64), (3, 2, 512, 64), (512, 8, 128, 64), (512, 8, 512, 256), (513, 8, 128, 64)])
 def test_moe_sort_forms(hip, t, k, E, chunk):
