@@ -497,7 +497,7 @@ hipError_t launch_gemv_f32(const float* w, int rows, int cols, const float* x, u
 // chain and many by the VALU (62 us for 4096 x 128 x 2048 at two instructions a term). Four forms by the work they leave a
 // CU (gemm_f32_form); router of 128 x 2048, us a call, before (one form: 4 chains a lane, x and weights
 // through one LDS buffer whose loads each step waited for) and now: 27 tokens 72 -> 18, 512 72 -> 29, 1501 72 -> 39,
-// 4096 77 -> 68. ----
+// 4096 77 -> 66. ----
 
 // A block of 4 waves takes 64 positions (a lane each) x 4 RW weight rows (RW chains a lane). x and the weight rows come
 // by direct global-to-LDS loads into a ring of gf_nb steps of 32 k (three or four steps in flight: one step's work is
